@@ -178,3 +178,43 @@ def test_invalid_nodes_are_rejected_on_the_host():
         bl[3] = l1[3]
         with pytest.raises(wsbb_amd.WsbbError):
             eng.bound(permT, l1, bl)
+
+
+@pytest.mark.parametrize("n,m", [(2, 2), (10, 3), (20, 24), (30, 7), (31, 8), (32, 9), (33, 12),
+                                 (62, 13), (63, 16), (64, 17), (65, 5), (94, 20), (95, 21), (96, 6),
+                                 (97, 4), (126, 10), (127, 11), (128, 3)])
+def test_lb2_matrix_core_operand_edges(n, m):
+    """Job counts at the edges of the 32-wide operands (two constant columns
+    after the jobs), machine counts at those of the padded rows, batches at
+    the tiles' edges, and times at 127, the largest the form takes; 128 and
+    126 + 2 jobs fall back to the scan.  Whole numbers: equal."""
+    rng = np.random.default_rng(n * 100 + m)
+    p = rng.integers(0, 128, size=(m, n)).astype(np.int32)
+    p[rng.integers(m), rng.integers(n)] = 127
+    big = p.copy()
+    big[0, 0] = 128
+    for q in (p, big):
+        o = oracle.Oracle(q)
+        with wsbb_amd.Engine(q) as eng:
+            for N in (1, 63, 129, 700):
+                permT, l1, l2 = batch_for(n, N, N)
+                ref = o.bound_batch(permT, l1, l2, kind=oracle.LB2, threads=8)
+                for groups in (1, 2, 4, 8):
+                    eng.set_launch(groups=groups)
+                    assert np.array_equal(eng.bound(permT, l1, l2), ref), (N, groups)
+
+
+@pytest.mark.parametrize("tid,N", [(51, 140_001), (71, 70_003), (21, 140_001)])
+def test_lb2_large_batches_in_several_launches(tid, N):
+    """Batches large enough for 128-node tiles (50 and 100 jobs) and one wave
+    per tile (20 jobs), whole and under a block cap."""
+    p = oracle.taillard(tid)[3]
+    n = p.shape[1]
+    permT, l1, l2 = wsbb_amd.random_nodes(n, N, 11)
+    idx = np.r_[0:200, N - 200:N, np.random.default_rng(5).choice(N, 3000, replace=False)]
+    ref = oracle.Oracle(p).bound_batch(permT[:, idx], l1[idx], l2[idx], threads=16)
+    with wsbb_amd.Engine(p) as eng:
+        got = eng.bound(permT, l1, l2)
+        eng.set_launch(groups=0, grid_blocks=100)
+        assert np.array_equal(eng.bound(permT, l1, l2), got)
+    assert np.array_equal(got[idx], ref)

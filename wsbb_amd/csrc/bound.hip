@@ -21,6 +21,8 @@
 // (heuristiqueCmax 64-77) and the tail combine (cmaxFin 92-100, 147-148).
 #include "bound.h"
 
+#include "johnson.h"
+
 #include <hip/hip_ext.h>
 
 #include <type_traits>
@@ -1224,6 +1226,12 @@ hipError_t launch_src(const DevTables& T, const Src& src, const BoundArgs& A,
                    : (bare && A.best == -1 && A.tile_sel == nullptr) ? 0
                    : (bare && A.best == -1 && A.margin < 0)          ? 3
                                                                      : 1;
+  if constexpr (Src::kState) {
+    if ((mode == 0 || mode == 3) && A.mfma && T.mf != nullptr && src.has_state())
+      return launch_johnson(T, src, A, grid_cap, stream);
+  } else {
+    if (mode == 0 && A.mfma && T.mf != nullptr) return launch_johnson(T, src, A, grid_cap, stream);
+  }
   // 8 or 16 waves per tile (1024-thread blocks) for small batches; the lean
   // variants for up to 16 machines fit four such waves per SIMD
   if (mode == 0 && A.best == -1 && T.steps16 != nullptr && A.groups <= 4 && A.pk != 0)

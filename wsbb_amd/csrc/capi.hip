@@ -11,6 +11,7 @@
 #include "../../include/wsbb_amd.h"
 #include "bound.h"
 #include "context.h"
+#include "johnson.h"
 
 namespace wsbb {
 
@@ -60,6 +61,19 @@ static uint8_t* scratch_of(int device) {
 }  // namespace wsbb
 
 using namespace wsbb;
+
+// The matrix-core form of LB2 holds times and time differences as signed
+// bytes and a pair's lag + p_a in two of them, and its columns (the jobs and
+// two constants) in four blocks of 32.
+static bool johnson_fits(const Instance& I) {
+  if (I.n + 2 > 128) return false;
+  for (int32_t v : I.p)
+    if (v > 127) return false;
+  for (int s = 0; s < I.P; ++s)
+    for (int j = 0; j < I.n; ++j)
+      if (I.lag[s * I.n + j] + I.p[I.pair_a[s] * I.n + j] > kXMax) return false;
+  return true;
+}
 
 int wsbb_ctx::groups_for(int N) const {
   if (launch.groups > 1) return launch.groups;
@@ -297,6 +311,19 @@ int wsbb_create(const int32_t* p, int n, int m, int device, wsbb_ctx** out) {
   T.Q0 = ctx->tables.as<const int32_t>(o_Q0);
   T.ptot = ctx->tables.as<const int32_t>(o_tot);
   T.steps16 = two16 ? ctx->tables.as<const uint2>(o_s16) : nullptr;
+  if (johnson_fits(I)) {
+    const size_t b_mf = johnson_bytes(n, m), b_pf = johnson_time_bytes(n);
+    if ((e = ctx->frags.reserve(b_mf + b_pf + 32 * size_t(n))) != hipSuccess) return fail(e, "hipMalloc(fragments)");
+    T.mf = ctx->frags.as<const int4>();
+    T.pf = ctx->frags.as<const int4>(b_mf);
+    T.pr = ctx->frags.as<const int4>(b_mf + b_pf);
+    if ((e = build_johnson(T, ctx->frags.as<int4>(), ctx->frags.as<int4>(b_mf),
+                           ctx->frags.as<int4>(b_mf + b_pf), ctx->stream)) != hipSuccess)
+      return fail(e, "fragment kernel launch");
+    // the tables are complete before any stream reads them (a mixed batch
+    // reads every instance's on one)
+    if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return fail(e, "hipStreamSynchronize");
+  }
   *out = ctx;
   return WSBB_OK;
 }
@@ -308,6 +335,7 @@ int wsbb_destroy(wsbb_ctx* ctx) {
   destroy_search(ctx);
   destroy_selector(ctx);
   ctx->tables.release();
+  ctx->frags.release();
   ctx->batch.release();
   if (ctx->ev_start) (void)hipEventDestroy(ctx->ev_start);
   if (ctx->ev_stop) (void)hipEventDestroy(ctx->ev_stop);
@@ -380,6 +408,7 @@ int wsbb_bound_batch_ex(wsbb_ctx* ctx, const uint8_t* permT, const int32_t* l1,
   A.best = best;
   A.groups = ctx->groups_for(N);
   A.pk = ctx->int16_for(N);
+  ctx->johnson_args(A);
   A.out = ctx->batch.as<int32_t>(o_out);
   A.argmax = argmax ? ctx->batch.as<int32_t>(o_am) : nullptr;
   A.pairv = pairv ? ctx->batch.as<int32_t>(o_pv) : nullptr;
@@ -490,6 +519,7 @@ int wsbb_bound_batch_noalloc(wsbb_ctx* ctx, const uint8_t* permT, const int32_t*
   A.best = best;
   A.groups = ctx->groups_for(N);
   A.pk = ctx->int16_for(N);
+  ctx->johnson_args(A);
   A.out = reinterpret_cast<int32_t*>(base + o_out);
   WSBB_HIP(launch_bound(ctx->T, src, A, ctx->grid_cap(), st), "bound kernel launch");
   WSBB_HIP(hipMemcpyAsync(out, A.out, size_t(4) * N, hipMemcpyDeviceToHost, st), "D2H out");
@@ -511,6 +541,7 @@ int wsbb_bound_device(wsbb_ctx* ctx, const uint8_t* d_permT, const int32_t* d_l1
   A.best = -1;
   A.groups = ctx->groups_for(N);
   A.pk = ctx->int16_for(N);
+  ctx->johnson_args(A);
   A.out = d_out;
   WSBB_HIP(launch_bound(ctx->T, src, A, ctx->grid_cap(), ctx->stream), "bound kernel launch");
   return WSBB_OK;
@@ -638,6 +669,7 @@ int wsbb_autotune(wsbb_ctx* ctx, int N, int reps, int32_t* shapes, float* ms,
       A.best = -1;
       A.groups = g;
       A.pk = ctx->int16_for(N);
+  ctx->johnson_args(A);
       A.out = static_cast<int32_t*>(dout);
       hipError_t e = launch_bound(ctx->T, src, A, grid, ctx->stream);  // warm-up
       if (e == hipSuccess) e = hipEventRecord(ctx->ev_start, ctx->stream);

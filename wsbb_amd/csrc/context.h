@@ -61,6 +61,7 @@ struct wsbb_ctx {
   wsbb::Instance inst;
   wsbb::DevTables T{};
   wsbb::DevBuf tables;  // every instance table in one allocation
+  wsbb::DevBuf frags;   // matrix-core operands of the instance (johnson.hip)
   wsbb::DevBuf batch;   // staging for host-buffer batch calls
   wsbb::Launch launch;
   int pool_capacity = 1 << 24;  // device node-pool capacity (nodes)
@@ -79,6 +80,16 @@ struct wsbb_ctx {
     return num_cus * 16;  // 16 blocks per CU: a 2^20-node batch, one per four tiles
   }
   int groups_for(int N) const;
+  // the matrix cores bound faster than either scan at every batch size; a
+  // caller who asks for the int16 form gets it
+  int mfma_for() const { return T.mf != nullptr && launch.int16 != 2; }
+  void johnson_args(wsbb::BoundArgs& A) const {
+    A.mfma = mfma_for();
+    A.num_cus = num_cus;
+    int tiles = (A.N + 63) / 64, cls = 0;  // as groups_for
+    while ((1 << (cls + 1)) <= tiles && cls < 31) ++cls;
+    A.waves = launch.groups > 1 ? launch.groups : tuned_groups[cls] > 0 ? tuned_groups[cls] : 0;
+  }
   // two nodes per lane pays once a batch gives every SIMD two 128-node tiles;
   // smaller launches are latency-bound and prefer more wavefronts
   int int16_for(long long N) const {

@@ -49,6 +49,11 @@ struct DevTables {
   const uint2* steps16;  // [P][n4] two-node form {job, (p_a - p_b mod 2^16)
                          // | (2^14 + lag + p_b) << 16}; pad = 0, plus 16
                          // zero steps; null when bound values may reach 2^14
+  const int4* mf;        // [P][row tiles][column blocks][64] matrix-core operands
+                         // of every pair's Johnson scan (johnson.hip), or null
+                         // when the instance's times do not fit them
+  const int4* pf;        // [column blocks][64] the processing times, alike
+  const int4* pr;        // [n] the processing times job-major, a byte each
 };
 
 // What a bound launch computes and where it writes.
@@ -74,6 +79,11 @@ struct BoundArgs {
   long long* stats;          // with tile_sel: [0] nodes, [1] full-LB2
                              // fallbacks, [2] node-pair evaluations
   int pk = 1;                // plain LB2 may run two nodes per lane (int16)
+  int waves = 0;             // johnson.hip: waves that split a tile's pairs
+                             // (1, 2 or 4), or 0: chosen by the launch
+  int num_cus = 256;
+  int mfma = 1;              // plain LB2 and tile subsets may run on the matrix
+                             // cores (johnson.hip) where the instance fits them
   // plain LB2 over pairs whose steps fit one scalar batch loads the next
   // pair's table lines ahead (set for launches of fewer waves than SIMDs,
   // where nothing else hides a scalar-cache miss)
@@ -157,6 +167,12 @@ struct BatchSource {
   __device__ __forceinline__ int slot(int k) const { return k; }
 };
 
+// a child's descriptor, limits and the one or two jobs it places
+struct Child {
+  int d, a, b, job, last;
+  bool two;
+};
+
 // Node source: children described by (parent, side, position) over a
 // position-major parent array (decompose_beginend child semantics).
 struct ChildSource {
@@ -180,7 +196,7 @@ struct ChildSource {
   const int32_t* hq = nullptr;
   const uint32_t* hm = nullptr;
   const int32_t* hw = nullptr;  // [MM][PN] work of the parent's scheduled jobs
-  __device__ __forceinline__ bool has_state() const { return hr != nullptr; }
+  __host__ __device__ __forceinline__ bool has_state() const { return hr != nullptr; }
   // heads, tails, scheduled mask and scheduled work of child k from its
   // parent's state; sp holds the processing times job-major in LDS
   __device__ __forceinline__ int key(int k) const { return desc[k]; }
@@ -247,6 +263,74 @@ struct ChildSource {
     stride = PN;
   }
   __device__ __forceinline__ int slot(int k) const { return k; }
+  // limits of the child with descriptor d
+  __device__ __forceinline__ void limits(int d, int& a, int& b) const {
+    const int par = d >> 9, side = (d >> 8) & 1;
+    a = pl1[par] + (side == 0);
+    b = pl2[par] - (side == 1);
+    if (b - a == 2) a += 1;
+  }
+  // a child in two parts: load_* issue the reads of its parent's state (heads
+  // and scheduled jobs, or tails) and of the jobs it places, place_* extend
+  // the state by them; row(j, pk) gives a job's times
+  __device__ __forceinline__ Child child(int d) const {
+    Child c;
+    c.d = d;
+    const int par = d >> 9, side = (d >> 8) & 1, j = d & 255;
+    const int pa = pl1[par], pb = pl2[par];
+    c.a = pa + (side == 0);
+    c.b = pb - (side == 1);
+    c.two = c.b - c.a == 2;
+    const uint8_t* col = ppermT + par;
+    c.job = col[static_cast<size_t>(j) * PN];  // placed at l1 + 1 or l2 - 1
+    c.last = 0;
+    if (c.two) {
+      // the last free job goes to the end of the prefix (limites_set)
+      c.last = perm_at(col, PN, side == 0 ? pa + 1 : pb - 1, j, c.a + 1);
+      c.a += 1;
+    }
+    return c;
+  }
+  template <int MM, class Set>
+  __device__ __forceinline__ void load_heads(const Child& c, int (&x)[MM], Set& set, int words) const {
+    const int par = c.d >> 9;
+#pragma unroll
+    for (int kk = 0; kk < MM; ++kk) x[kk] = hr[static_cast<size_t>(kk) * PN + par];
+    uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < words) w[i] = hm[static_cast<size_t>(i) * PN + par];
+    set.lo = w[0] | static_cast<unsigned long long>(w[1]) << 32;
+    set.hi = w[2] | static_cast<unsigned long long>(w[3]) << 32;
+  }
+  template <int MM>
+  __device__ __forceinline__ void load_tails(const Child& c, int (&y)[MM]) const {
+#pragma unroll
+    for (int kk = 0; kk < MM; ++kk) y[kk] = hq[static_cast<size_t>(kk) * PN + (c.d >> 9)];
+  }
+  template <int MM, class Set, class Row>
+  __device__ __forceinline__ void place_heads(const Child& c, int (&x)[MM], Set& set, Row row) const {
+    set.add(c.job);
+    if (((c.d >> 8) & 1) == 0) {
+      int pk[MM];
+      row(c.job, pk);
+      head_step<MM>(x, pk);
+    }
+    if (c.two) {
+      int pk[MM];
+      row(c.last, pk);
+      set.add(c.last);
+      head_step<MM>(x, pk);
+    }
+  }
+  template <int MM, class Row>
+  __device__ __forceinline__ void place_tails(const Child& c, int (&y)[MM], Row row) const {
+    if ((c.d >> 8) & 1) {
+      int pk[MM];
+      row(c.job, pk);
+      tail_step<MM>(y, pk);
+    }
+  }
 };
 
 // Node source: the children listed in list[0..*count) (a compacted subset of
@@ -258,7 +342,7 @@ struct ListSource {
   ChildSource base;
   const int32_t* list;
   const int* count;
-  __device__ __forceinline__ bool has_state() const { return base.has_state(); }
+  __host__ __device__ __forceinline__ bool has_state() const { return base.has_state(); }
   template <int MM, int NW>
   __device__ __forceinline__ void state(int k, const int32_t* sp, int (&r)[MM], int (&q)[MM],
                                         uint32_t (&sm)[NW], int (&sc)[MM]) const {

@@ -1549,7 +1549,7 @@ static hipError_t launch_round(wsbb_ctx* ctx, const SArgs& A, int kind, hipEvent
   // parent state for the int32 bound kernel (learned subsets, logging,
   // rounds below the two-node form's batch size); the two-node form of plain
   // LB2 runs its own recurrences
-  const bool pk_round = kind == WSBB_LB2 && selector_log_stride(ctx) == 0 &&
+  const bool pk_round = kind == WSBB_LB2 && selector_log_stride(ctx) == 0 && !ctx->mfma_for() &&
                         ctx->T.steps16 != nullptr && ctx->int16_for(A.CCAP);
   const bool want_state = !pk_round;
   // per-parent selector features come from expand when m is a multiple of
@@ -1600,6 +1600,7 @@ static hipError_t launch_round(wsbb_ctx* ctx, const SArgs& A, int kind, hipEvent
   B.out = A.c_bound;
   B.feat_scale = static_cast<float>(ctx->inst.path_bound);
   B.pk = ctx->int16_for(A.CCAP);
+  ctx->johnson_args(B);
   const BatchSource parents{A.p_perm, A.p_l1, A.p_l2, A.PCAP};
   const float fscale = static_cast<float>(ctx->inst.path_bound);
   if (kind == WSBB_LEARNED) {
@@ -1659,6 +1660,7 @@ static hipError_t launch_round(wsbb_ctx* ctx, const SArgs& A, int kind, hipEvent
     Bf.margin = -1;
     Bf.out = A.c_bound;
     Bf.pk = ctx->int16_for(A.CCAP);
+    ctx->johnson_args(Bf);
     if ((e = launch_bound(ctx->T, ls, Bf, ctx->grid_cap(), st)) != hipSuccess) return e;
     hipLaunchKernelGGL(k_fallback_stats, dim3(1), dim3(1), 0, st, A);
   }
