@@ -118,6 +118,27 @@ __device__ __forceinline__ void job_row(const int32_t* sp, int j, int (&pk)[MM])
   }
 }
 
+// row i of a global [][MM] array, four words a load (and store)
+template <int MM>
+__device__ __forceinline__ void load_row(const int32_t* a, int i, int (&v)[MM]) {
+  const int4* q = reinterpret_cast<const int4*>(a) + static_cast<size_t>(i) * (MM / 4);
+#pragma unroll
+  for (int k4 = 0; k4 < MM / 4; ++k4) {
+    const int4 x = q[k4];
+    v[4 * k4] = x.x;
+    v[4 * k4 + 1] = x.y;
+    v[4 * k4 + 2] = x.z;
+    v[4 * k4 + 3] = x.w;
+  }
+}
+template <int MM>
+__device__ __forceinline__ void store_row(int32_t* a, int i, const int (&v)[MM]) {
+  int4* q = reinterpret_cast<int4*>(a) + static_cast<size_t>(i) * (MM / 4);
+#pragma unroll
+  for (int k4 = 0; k4 < MM / 4; ++k4)
+    q[k4] = make_int4(v[4 * k4], v[4 * k4 + 1], v[4 * k4 + 2], v[4 * k4 + 3]);
+}
+
 template <int NW>
 __device__ __forceinline__ void set_job_bit(uint32_t (&sm)[NW], int j) {
 #pragma unroll
@@ -189,13 +210,13 @@ struct ChildSource {
   const int32_t* pl2;
   const int32_t* desc;    // [N] parent << 9 | side << 8 | j
   int PN, N;
-  // optional parent state (heads [MM][PN], tails [MM][PN] of the parent's
+  // optional parent state (heads [PN][MM], tails [PN][MM] of the parent's
   // prefix and suffix, scheduled-job masks [NW][PN]): a child's heads and
   // tails are then its parent's extended by the one or two jobs it places
   const int32_t* hr = nullptr;
   const int32_t* hq = nullptr;
   const uint32_t* hm = nullptr;
-  const int32_t* hw = nullptr;  // [MM][PN] work of the parent's scheduled jobs
+  const int32_t* hw = nullptr;  // [PN][MM] work of the parent's scheduled jobs
   __host__ __device__ __forceinline__ bool has_state() const { return hr != nullptr; }
   // heads, tails, scheduled mask and scheduled work of child k from its
   // parent's state; sp holds the processing times job-major in LDS
@@ -211,12 +232,9 @@ struct ChildSource {
                                             uint32_t (&sm)[NW], int (&sc)[MM]) const {
     const int par = d >> 9, side = (d >> 8) & 1, j = d & 255;
     const int pa = pl1[par], pb = pl2[par];
-#pragma unroll
-    for (int kk = 0; kk < MM; ++kk) {
-      r[kk] = hr[static_cast<size_t>(kk) * PN + par];
-      q[kk] = hq[static_cast<size_t>(kk) * PN + par];
-      sc[kk] = hw[static_cast<size_t>(kk) * PN + par];
-    }
+    load_row<MM>(hr, par, r);
+    load_row<MM>(hq, par, q);
+    load_row<MM>(hw, par, sc);
 #pragma unroll
     for (int w = 0; w < NW; ++w) sm[w] = hm[static_cast<size_t>(w) * PN + par];
     const uint8_t* col = ppermT + par;
@@ -294,8 +312,7 @@ struct ChildSource {
   template <int MM, class Set>
   __device__ __forceinline__ void load_heads(const Child& c, int (&x)[MM], Set& set, int words) const {
     const int par = c.d >> 9;
-#pragma unroll
-    for (int kk = 0; kk < MM; ++kk) x[kk] = hr[static_cast<size_t>(kk) * PN + par];
+    load_row<MM>(hr, par, x);
     uint32_t w[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -305,8 +322,7 @@ struct ChildSource {
   }
   template <int MM>
   __device__ __forceinline__ void load_tails(const Child& c, int (&y)[MM]) const {
-#pragma unroll
-    for (int kk = 0; kk < MM; ++kk) y[kk] = hq[static_cast<size_t>(kk) * PN + (c.d >> 9)];
+    load_row<MM>(hq, c.d >> 9, y);
   }
   template <int MM, class Set, class Row>
   __device__ __forceinline__ void place_heads(const Child& c, int (&x)[MM], Set& set, Row row) const {

@@ -35,6 +35,7 @@ struct JohnsonShape {
   int tpb;         // tiles per block
   int tile_bytes;  // LDS of one tile
   int first_block; // of this launch
+  int list_rows;   // 64-word rows of a tile's pair list
   const int* list; // the children to bound, or null: all of them
 };
 

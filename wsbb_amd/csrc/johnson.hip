@@ -559,44 +559,66 @@ __global__ __launch_bounds__(256, (NB == 2 && KB <= 2 ? 3 : 2)) void k_johnson(D
     bool suf[NB];
 #pragma unroll
     for (int c = 0; c < NB; ++c) suf[c] = __shfl(l2[c >> 1], 32 * (c & 1) + col, 64) < n;
-    // the set bits of the tile's mask words in order, one pair ahead: its
-    // fragments are loaded while the pair before it is multiplied
-    int wd = 0;
-    uint32_t word = ld_const_u32(tsel, 0);
-    auto pick = [&]() {
-      while (word == 0) {
-        if (++wd >= A.nsw) return -1;
-        word = ld_const_u32(tsel, wd);
+    // the tile's pairs as a list in LDS, one word each: entry, first and
+    // second machine (all waves of the tile write the same list)
+    uint32_t* list = reinterpret_cast<uint32_t*>(lds + L.total) + tib * 64 * H.list_rows;
+    int np = 0;
+    for (int s0 = 0; s0 < T.P; s0 += 64) {
+      const int s = s0 + lane;
+      const bool take = s < T.P && ((tsel[s >> 5] >> (s & 31)) & 1u);
+      const unsigned long long bal = __ballot(take);
+      if (take) {
+        const int2 ab = T.pairs[s];
+        const int e = 2 * johnson_first_couple(m, ab.x) + ab.y - ab.x - 1;
+        list[np + __popcll(bal & ((1ull << lane) - 1ull))] =
+            static_cast<uint32_t>(e) | (ab.x << 16) | (ab.y << 24);
       }
-      const int s = 32 * wd + __builtin_ctz(word);
-      word &= word - 1;
-      return s < T.P ? s : -1;
-    };
-    auto fragments = [&](int s) {
-      // the entry of pair s = (x, y): its couple, then its place in it
-      const int2 xy = ld_const2(T.pairs, s);
-      const int e = 2 * johnson_first_couple(m, xy.x) + xy.y - xy.x - 1;
-      return reinterpret_cast<const char*>(T.mf) + (static_cast<size_t>(e) * rts + rt) * KB * 1024;
-    };
-    int s = pick();
-    if (s >= 0) fetch(fragments(s), a[0]);
-    while (s >= 0) {
-      const int2 ab = ld_const2(T.pairs, s);
-      const int sn = pick();
-      fetch(fragments(sn >= 0 ? sn : s), a[1]);
+      np += __popcll(bal);
+    }
+    np = __builtin_amdgcn_readfirstlane(np);
+    if (np > 0) {
+      // two pairs ahead (a rolled loop: unrolled, four pairs' products were
+      // in registers at once and spilled)
+      v4i f[3][KB];
+      uint32_t w[3];
+      auto ask = [&](int i, uint32_t& word, v4i(&v)[KB]) {
+        word = __builtin_amdgcn_readfirstlane(list[min(i, np - 1)]);
+        fetch(reinterpret_cast<const char*>(T.mf) +
+                  (static_cast<size_t>(word & 0xffffu) * rts + rt) * KB * 1024,
+              v);
+      };
+      ask(0, w[0], f[0]);
+      ask(1, w[1], f[1]);
+#pragma unroll 1
+      for (int i = 0; i < np; ++i) {
+        ask(i + 2, w[2], f[2]);
+        const int xa = (w[0] >> 16) & 0xff, xb = w[0] >> 24;
+        int sa[NB], sb[NB], ea[NB], eb[NB];
 #pragma unroll
-      for (int c = 0; c < NB; ++c) {
-        v16i z = mfma_i8(a[0][0], B[c][0], C[c]);
+        for (int c = 0; c < NB; ++c) {
+          sa[c] = stc[xa * TN + 32 * c];
+          sb[c] = stc[xb * TN + 32 * c];
+          ea[c] = ewc[xa * TN + 32 * c];
+          eb[c] = ewc[xb * TN + 32 * c];
+        }
+        v16i z[NB];
 #pragma unroll
-        for (int kb = 1; kb < KB; ++kb) z = mfma_i8(a[0][kb], B[c][kb], z);
-        const int sa = stc[ab.x * TN + 32 * c], sb = stc[ab.y * TN + 32 * c];
-        const int ea = ewc[ab.x * TN + 32 * c], eb = ewc[ab.y * TN + 32 * c];
-        const int v = max(max_rows<NR>(z) + sa, sb) + eb;
-        lb[c] = max(lb[c], max(v, suf[c] ? sa + ea : 0));
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+          for (int c = 0; c < NB; ++c) z[c] = mfma_i8(f[0][kb], B[c][kb], kb == 0 ? C[c] : z[c]);
+#pragma unroll
+        for (int c = 0; c < NB; ++c) {
+          const int v = max(max_rows<NR>(z[c]) + sa[c], sb[c]) + eb[c];
+          lb[c] = max(lb[c], max(v, suf[c] ? sa[c] + ea[c] : 0));
+        }
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          f[0][kb] = f[1][kb];
+          f[1][kb] = f[2][kb];
+        }
+        w[0] = w[1];
+        w[1] = w[2];
       }
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) a[0][kb] = a[1][kb];
-      s = sn;
     }
   } else {
     // row offsets of the couple's machines
@@ -720,7 +742,9 @@ hipError_t launch_kernel(const DevTables& T, const Src& src, const BoundArgs& A,
   const int body = std::max(Src::kState ? 0 : T.n * TN, 2 * MM * TN * 4);
   H.tile_bytes = ((body + 15) & ~15) + 2 * H.rts * TN * 4;
   const int nodes = TN * H.tpb;
-  const size_t shmem = Layout(H.tpb, H.tile_bytes, waves, nodes, T.n, rs).total;
+  H.list_rows = (T.P + 63) / 64;
+  const size_t shmem = Layout(H.tpb, H.tile_bytes, waves, nodes, T.n, rs).total +
+                       (SUBSET ? 256 * H.list_rows * H.tpb : 0);
   const int blocks = (A.N + nodes - 1) / nodes;
   // a block bounds its tiles and ends (a loop over tiles kept the whole
   // prologue's constants in registers); more blocks than the cap run as

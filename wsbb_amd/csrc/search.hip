@@ -119,10 +119,10 @@ struct SArgs {
   int* r_order;     // [PCAP][n] per parent, by rank: the chosen-side child index
   int* r_cost;      // [PCAP][n] per parent, by rank: that child's bound
   int* r_leaves;    // [kRankGrid] leaf children counted by each rank block
-  int* p_hr;        // [MM][PCAP + 1] heads of the parent's prefix
-  int* p_hq;        // [MM][PCAP + 1] tails of the parent's suffix
+  int* p_hr;        // [PCAP + 1][MM] heads of the parent's prefix
+  int* p_hq;        // [PCAP + 1][MM] tails of the parent's suffix
   uint32_t* p_hm;   // [NW][PCAP + 1] the parent's scheduled jobs
-  int* p_hw;        // [MM][PCAP + 1] work of the parent's scheduled jobs
+  int* p_hw;        // [PCAP + 1][MM] work of the parent's scheduled jobs
   // selector features of the parents written by expand (m a multiple of
   // four): BF16 MFMA fragments and/or FP32 rows [5m][x_ld], or null
   uint2* x_frag;
@@ -679,7 +679,7 @@ __global__ __launch_bounds__(kExpandBlock) void k_expand(SArgs S, DevTables T, i
   __syncthreads();
   const int n = S.n, m = S.m, P = S.P;
   const int lane = threadIdx.x & 63;
-  const size_t PH = static_cast<size_t>(S.PCAP);  // rows of the parent state, as ChildSource reads them
+  const size_t PH = static_cast<size_t>(S.PCAP);  // rows of the scheduled jobs, as ChildSource reads them
   long long work = 0;
   if (mine_p) {
     const int l1 = S.s_l1[si], l2 = S.s_l2[si], cost = S.s_cost[si];
@@ -747,12 +747,9 @@ __global__ __launch_bounds__(kExpandBlock) void k_expand(SArgs S, DevTables T, i
 #pragma unroll
         for (int k = 0; k < MM; ++k) wk[k] += pk[k];
       }
-#pragma unroll
-      for (int k = 0; k < MM; ++k) {
-        S.p_hr[k * PH + p] = r[k];
-        S.p_hq[k * PH + p] = q[k];
-        S.p_hw[k * PH + p] = wk[k];
-      }
+      store_row<MM>(S.p_hr, p, r);
+      store_row<MM>(S.p_hq, p, q);
+      store_row<MM>(S.p_hw, p, wk);
 #pragma unroll
       for (int w = 0; w < NW; ++w) S.p_hm[w * PH + p] = sm[w];
       // selector features of the parent (the feature kernel's definition and
