@@ -347,3 +347,27 @@ def test_online_training_resumes_to_the_optimum():
     assert after < 0.3 * 190 * (rs["bounded"] - fs["bounded"])
     print(f"plain {ps['bounded']} nodes; online {rs['bounded']} nodes, "
           f"{after / max(rs['bounded'] - fs['bounded'], 1):.1f} pairs per node after the switch")
+
+
+@pytest.mark.parametrize("m,B", [(2, 1), (5, 7), (12, 8), (13, 257), (24, 513)])
+def test_gradients_at_batch_and_size_edges(m, B):
+    """Batches around the row blocks (8) and the weight-gradient chunks (256),
+    machine counts from one pair to the most, against torch in float32 on
+    the same BF16-rounded weights and inputs; what is left is the hidden
+    activations' rounding, which a sum in another order can flip (one BF16
+    step in a sum over 128): tolerances as in test_gradients_match_torch."""
+    p = np.random.default_rng(m).integers(1, 100, size=(m, 20)).astype(np.int32)
+    with wsbb_amd.Engine(p) as eng:
+        eng.selector_init(seed=4)
+        params = eng.selector_params()
+        feat, label = random_records(eng, B + 5, 7)
+        eng.selector_set_records(feat, label)
+        idx = np.random.default_rng(8).permutation(B + 5)[:B].astype(np.int32)
+        loss, g = eng.selector_grad(idx)
+        again, _ = eng.selector_grad(idx)
+    tloss, tg = torch_grads(params, feat, label, idx)
+    assert loss == again
+    assert abs(loss - tloss) <= 1e-3 * abs(tloss) + 1e-6
+    for k in ("W1", "b1", "W2", "b2"):
+        scale = np.abs(tg[k]).max()
+        assert np.allclose(g[k], tg[k], rtol=0, atol=2e-2 * scale + 1e-12), k

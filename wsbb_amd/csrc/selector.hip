@@ -383,166 +383,238 @@ struct TrainArgs {
   int ldf;
   const int* label;        // [records]
   const int* idx;          // [B] record index of each row
-  const float* W1;         // [F][128] masters
-  const float* b1;
-  const float* W2;         // [128][P]
+  const float* b1;         // masters
   const float* b2;
   float* X;                // [B][F] bf16-rounded inputs
-  float* A1;               // [B][128] pre-activations
   float* Hb;               // [B][128] bf16-rounded activations
-  float* Z;                // [B][P]
   float* dZ;               // [B][P]
   float* dH;               // [B][128]
   float* loss;             // [B]
-  float* gW1;
-  float* gb1;
-  float* gW2;
-  float* gb2;
   int nvalid;              // rows with a label (>= 0)
-  float* part;             // split-K partial sums of the weight gradients
+  float* part;             // [splits][129][P], then [splits][F + 1][128] partial sums
+                           // of the weight gradients
+  float* W1r;              // [F][128] W1 rounded to BF16
+  float* W2r;              // [128][P] W2 rounded to BF16
+  float* W2t;              // [P][128] the same, transposed
 };
 
 // Weight gradients are batch reductions C[m][n] = sum_b A[b][m] Bm[b][n]
 // (A = activations or inputs, Bm = output gradients), with an implicit row
-// m = M of ones in A so that C[M][n] is the bias gradient.  64 x 64 output
-// tiles, the batch split into chunks of kWgradK rows (one block each) that
-// stage 32-row slices of A and Bm in LDS; each thread accumulates a 4 x 4
-// block.  Partial sums go to part[split][M + 1][N] and are added in split
-// order by k_tr_wreduce, so the result does not depend on timing.
+// m = M of ones in A so that C[M][n] is the bias gradient.  The batch is
+// split into chunks of kWgradK rows; a chunk's sums run in row order and the
+// chunks are added in order (k_tr_update), so the result does not depend on
+// timing or on how the output is tiled.
+//
+// Both products in one launch, 32 x 32 outputs a block: 64 x 64 tiles left a
+// minibatch of 2048 with 72 blocks, and each waited for its eight 32-row
+// slices in turn.  Here a block loads 128 rows of both operands at once; 256
+// to 500 blocks (20x20: 55 us a product before, 13 us for both).
 constexpr int kWgradK = 256;
+constexpr int kWgradT = 32;   // output tile
+constexpr int kWgradS = 128;  // rows staged at once
 
-__global__ __launch_bounds__(256) void k_tr_wgrad(const float* A, int M, const float* Bm, int N,
-                                                  int K, float* part) {
-  __shared__ float As[32][68];
-  __shared__ float Bs[32][68];
+__host__ __device__ inline int wgrad_tiles(int M, int N) {
+  return ((M + 1 + kWgradT - 1) / kWgradT) * ((N + kWgradT - 1) / kWgradT);
+}
+
+__global__ __launch_bounds__(256) void k_tr_wgrad(TrainArgs T) {
+  __shared__ float As[kWgradS][kWgradT + 2];
+  __shared__ float Bs[kWgradS][kWgradT + 2];
   const int t = threadIdx.x, ty = t >> 4, tx = t & 15;
-  const int m0 = blockIdx.x * 64, n0 = blockIdx.y * 64, split = blockIdx.z;
-  const int kb = split * kWgradK, ke = min(kb + kWgradK, K);
-  float acc[4][4];
+  const int split = blockIdx.y, splits = gridDim.y;
+  // tiles of gW2 = Hb^T dZ, then of gW1 = X^T dH
+  int tile = blockIdx.x;
+  const int tiles2 = wgrad_tiles(kHidden, T.P);
+  const bool second = tile >= tiles2;
+  if (second) tile -= tiles2;
+  const float* A = second ? T.X : T.Hb;
+  const float* Bm = second ? T.dH : T.dZ;
+  const int M = second ? T.F : kHidden, N = second ? kHidden : T.P;
+  float* part = T.part + (second ? static_cast<size_t>(splits) * (kHidden + 1) * T.P : 0);
+  const int tn = (N + kWgradT - 1) / kWgradT;
+  const int m0 = tile / tn * kWgradT, n0 = tile % tn * kWgradT;
+  const int kb = split * kWgradK, ke = min(kb + kWgradK, T.B);
+  float acc[2][2] = {};
+  for (int k0 = kb; k0 < ke; k0 += kWgradS) {
+    float va[16], vb[16];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int r = 0; r < 16; ++r) {
+      // clamped: every load is issued before the first is used
+      const int kk = min(k0 + 8 * r + (t >> 5), ke - 1);
+      va[r] = A[static_cast<size_t>(kk) * M + min(m0 + (t & 31), M - 1)];
+      vb[r] = Bm[static_cast<size_t>(kk) * N + min(n0 + (t & 31), N - 1)];
+    }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-  for (int k0 = kb; k0 < ke; k0 += 32) {
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int e = t + 256 * r, k = e >> 6, c = e & 63;
-      const int kk = k0 + k, m = m0 + c, n = n0 + c;
-      const bool kin = kk < ke;
-      As[k][c] = !kin ? 0.f : m < M ? A[static_cast<size_t>(kk) * M + m] : (m == M ? 1.f : 0.f);
-      Bs[k][c] = kin && n < N ? Bm[static_cast<size_t>(kk) * N + n] : 0.f;
+    for (int r = 0; r < 16; ++r) {
+      As[8 * r + (t >> 5)][t & 31] = m0 + (t & 31) < M ? va[r] : 1.f;
+      Bs[8 * r + (t >> 5)][t & 31] = vb[r];
     }
     __syncthreads();
+    const int cnt = min(kWgradS, ke - k0);
 #pragma unroll 8
-    for (int k = 0; k < 32; ++k) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[k][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = Bs[k][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
+    for (int k = 0; k < cnt; ++k) {
+      const float a0 = As[k][2 * ty], a1 = As[k][2 * ty + 1];
+      const float b0 = Bs[k][2 * tx], b1 = Bs[k][2 * tx + 1];
+      acc[0][0] = fmaf(a0, b0, acc[0][0]);
+      acc[0][1] = fmaf(a0, b1, acc[0][1]);
+      acc[1][0] = fmaf(a1, b0, acc[1][0]);
+      acc[1][1] = fmaf(a1, b1, acc[1][1]);
     }
     __syncthreads();
   }
   float* out = part + static_cast<size_t>(split) * (M + 1) * N;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
-    if (m > M) continue;
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n < N) out[static_cast<size_t>(m) * N + n] = acc[i][j];
+    for (int j = 0; j < 2; ++j) {
+      const int m = m0 + 2 * ty + i, n = n0 + 2 * tx + j;
+      if (m <= M && n < N) out[static_cast<size_t>(m) * N + n] = acc[i][j];
     }
+}
+
+// Forward and backward of kTrainRows records a block, from the gathered
+// features to the gradient of the hidden pre-activations: one pass instead of
+// five launches that read and wrote the batch's activations and, per output,
+// rounded every weight again (20x20, 2048 records: 95 us before, 24 us).  The
+// weights come rounded to BF16 (W1r, W2r, and W2t for the backward product);
+// each sum runs over its index in order, one thread per output.
+constexpr int kTrainRows = 8, kTrainThreads = 512;  // a wave per row in the softmax
+constexpr int kMaxFeat = 5 * kMaxMachines;
+constexpr int kMaxPairs = kMaxMachines * (kMaxMachines - 1) / 2;
+
+__global__ __launch_bounds__(kTrainThreads) void k_tr_rows(TrainArgs T) {
+  constexpr int R = kTrainRows, ZP = kMaxPairs + 4;
+  __shared__ __align__(16) float xs[kMaxFeat][R];
+  __shared__ __align__(16) float hs[kHidden][R];
+  __shared__ __align__(16) float zs[R][ZP];  // outputs, then their gradients
+  const int t = threadIdx.x, b0 = blockIdx.x * R;
+  const int F = T.F, P = T.P;
+  for (int i = t; i < F * R; i += kTrainThreads) {
+    const int f = i / R, r = i % R, b = b0 + r;
+    float x = 0.f;
+    if (b < T.B) {
+      x = bfround(T.feat[static_cast<size_t>(f) * T.ldf + T.idx[b]]);
+      T.X[static_cast<size_t>(b) * F + f] = x;
+    }
+    xs[f][r] = x;
+  }
+  __syncthreads();
+  // hidden unit h of rows r0, r0 + 1
+  const int h = t & (kHidden - 1), r0 = 2 * (t / kHidden);
+  float pre[2] = {0.f, 0.f};
+#pragma unroll 10
+  for (int f = 0; f < F; ++f) {
+    const float w = T.W1r[f * kHidden + h];
+    const float2 x = *reinterpret_cast<const float2*>(&xs[f][r0]);
+    pre[0] = fmaf(x.x, w, pre[0]);
+    pre[1] = fmaf(x.y, w, pre[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    pre[i] += T.b1[h];
+    const float v = bfround(fmaxf(pre[i], 0.f));
+    hs[h][r0 + i] = v;
+    if (b0 + r0 + i < T.B) T.Hb[static_cast<size_t>(b0 + r0 + i) * kHidden + h] = v;
+  }
+  __syncthreads();
+  // output s of rows q0 .. q0 + 3
+  const int q0 = 4 * (t >> 8);
+  for (int s = t & 255; s < P; s += 256) {
+    float z[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 16
+    for (int k = 0; k < kHidden; ++k) {
+      const float w = T.W2r[k * P + s];
+      const float4 p = *reinterpret_cast<const float4*>(&hs[k][q0]);
+      z[0] = fmaf(p.x, w, z[0]);
+      z[1] = fmaf(p.y, w, z[1]);
+      z[2] = fmaf(p.z, w, z[2]);
+      z[3] = fmaf(p.w, w, z[3]);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) zs[q0 + r][s] = z[r] + T.b2[s];
+  }
+  __syncthreads();
+  // one wave per row: lanes over the pairs, wave reductions for max and sum
+  const int wave = t >> 6, lane = t & 63;
+  {
+    const int r = wave;
+    const int b = b0 + r;
+    const int y = b < T.B ? T.label[T.idx[b]] : -1;
+    float* z = zs[r];
+    if (y < 0) {
+      for (int s = lane; s < P; s += 64) z[s] = 0.f;
+      if (lane == 0 && b < T.B) T.loss[b] = 0.f;
+    } else {
+      const float zy = z[y];
+      float mx = -INFINITY;
+      for (int s = lane; s < P; s += 64) mx = fmaxf(mx, z[s]);
+      for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
+      float sum = 0.f;
+      for (int s = lane; s < P; s += 64) sum += expf(z[s] - mx);
+      for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+      const float inv = 1.f / sum, scale = 1.f / static_cast<float>(T.nvalid);
+      for (int s = lane; s < P; s += 64)
+        z[s] = (expf(z[s] - mx) * inv - (s == y ? 1.f : 0.f)) * scale;
+      if (lane == 0) T.loss[b] = (logf(sum) + mx - zy) * scale;
+    }
+    if (b < T.B)
+      for (int s = lane; s < P; s += 64) T.dZ[static_cast<size_t>(b) * P + s] = z[s];
+  }
+  __syncthreads();
+  float g[2] = {0.f, 0.f};
+#pragma unroll 10
+  for (int s = 0; s < P; ++s) {
+    const float w = T.W2t[s * kHidden + h];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) g[i] = fmaf(zs[r0 + i][s], w, g[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    if (b0 + r0 + i < T.B)
+      T.dH[static_cast<size_t>(b0 + r0 + i) * kHidden + h] = pre[i] > 0.f ? g[i] : 0.f;
+}
+
+// parameter i's weight as the products read it: rounded, W2 also transposed
+__device__ __forceinline__ void put_rounded(const TrainArgs& T, int i, float w) {
+  if (i < T.F * kHidden) T.W1r[i] = bfround(w);
+  const int j = i - (T.F + 1) * kHidden;
+  if (j >= 0 && j < kHidden * T.P) {
+    const float v = bfround(w);
+    T.W2r[j] = v;
+    T.W2t[(j % T.P) * kHidden + j / T.P] = v;
   }
 }
-
-// C = sum over splits; rows 0..M-1 to W, row M to the bias gradient
-__global__ void k_tr_wreduce(const float* part, int M, int N, int splits, float* W, float* bias) {
+__global__ void k_tr_round(TrainArgs T, const float* w, int np) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int tot = (M + 1) * N;
-  if (i >= tot) return;
-  float g = 0.f;
-  for (int sp = 0; sp < splits; ++sp) g += part[static_cast<size_t>(sp) * tot + i];
-  if (i < M * N)
-    W[i] = g;
-  else
-    bias[i - M * N] = g;
+  if (i < np) put_rounded(T, i, w[i]);
 }
 
-__global__ void k_tr_in(TrainArgs T) {
+// Parameter i (W1, b1, W2, b2 in one array): its gradient, the splits added
+// in order, then the Adam step (ADAM), or the gradient itself.
+template <bool ADAM>
+__global__ void k_tr_update(TrainArgs T, float* w, float* m, float* v, float* g, int np, int splits,
+                            float lr, float b1c, float b2c) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= T.B * T.F) return;
-  const int b = i / T.F, f = i - b * T.F;
-  T.X[i] = bfround(T.feat[static_cast<size_t>(f) * T.ldf + T.idx[b]]);
-}
-
-__global__ void k_tr_hidden(TrainArgs T) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= T.B * kHidden) return;
-  const int b = i / kHidden, h = i - b * kHidden;
-  float a = 0.f;
-  for (int f = 0; f < T.F; ++f) a += T.X[b * T.F + f] * bfround(T.W1[f * kHidden + h]);
-  a += T.b1[h];
-  T.A1[i] = a;
-  T.Hb[i] = bfround(fmaxf(a, 0.f));
-}
-
-__global__ void k_tr_out(TrainArgs T) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= T.B * T.P) return;
-  const int b = i / T.P, s = i - b * T.P;
-  float z = 0.f;
-  for (int h = 0; h < kHidden; ++h) z += T.Hb[b * kHidden + h] * bfround(T.W2[h * T.P + s]);
-  T.Z[i] = z + T.b2[s];
-}
-
-// one wave per row: lanes over the pairs, wave reductions for max and sum
-__global__ __launch_bounds__(256) void k_tr_softmax(TrainArgs T) {
-  const int b = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (b >= T.B) return;
-  const int y = T.label[T.idx[b]];
-  const float* z = T.Z + static_cast<size_t>(b) * T.P;
-  float* dz = T.dZ + static_cast<size_t>(b) * T.P;
-  if (y < 0) {
-    for (int s = lane; s < T.P; s += 64) dz[s] = 0.f;
-    if (lane == 0) T.loss[b] = 0.f;
-    return;
+  if (i >= np) return;
+  const int tot1 = (T.F + 1) * kHidden, tot2 = (kHidden + 1) * T.P;
+  const bool first = i < tot1;
+  const float* part = first ? T.part + static_cast<size_t>(splits) * tot2 + i : T.part + (i - tot1);
+  const int step = first ? tot1 : tot2;
+  float gi = 0.f;
+#pragma unroll 8
+  for (int sp = 0; sp < splits; ++sp) gi += part[static_cast<size_t>(sp) * step];
+  if constexpr (!ADAM) {
+    g[i] = gi;
+  } else {
+    const float beta1 = 0.9f, beta2 = 0.999f, eps = 1e-8f;
+    const float mi = beta1 * m[i] + (1.f - beta1) * gi;
+    const float vi = beta2 * v[i] + (1.f - beta2) * gi * gi;
+    m[i] = mi;
+    v[i] = vi;
+    const float wi = w[i] - lr * (mi / b1c) / (sqrtf(vi / b2c) + eps);
+    w[i] = wi;
+    put_rounded(T, i, wi);
   }
-  float mx = -INFINITY;
-  for (int s = lane; s < T.P; s += 64) mx = fmaxf(mx, z[s]);
-  for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
-  float sum = 0.f;
-  for (int s = lane; s < T.P; s += 64) sum += expf(z[s] - mx);
-  for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
-  const float inv = 1.f / sum, scale = 1.f / static_cast<float>(T.nvalid);
-  for (int s = lane; s < T.P; s += 64) dz[s] = (expf(z[s] - mx) * inv - (s == y ? 1.f : 0.f)) * scale;
-  if (lane == 0) T.loss[b] = (logf(sum) + mx - z[y]) * scale;
-}
-
-__global__ void k_tr_dH(TrainArgs T) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= T.B * kHidden) return;
-  const int b = i / kHidden, h = i - b * kHidden;
-  float g = 0.f;
-  if (T.A1[i] > 0.f)
-    for (int s = 0; s < T.P; ++s) g += T.dZ[static_cast<size_t>(b) * T.P + s] * bfround(T.W2[h * T.P + s]);
-  T.dH[i] = g;
-}
-
-__global__ void k_adam(float* w, float* m, float* v, const float* g, int n, float lr,
-                       float b1c, float b2c) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float beta1 = 0.9f, beta2 = 0.999f, eps = 1e-8f;
-  const float mi = beta1 * m[i] + (1.f - beta1) * g[i];
-  const float vi = beta2 * v[i] + (1.f - beta2) * g[i] * g[i];
-  m[i] = mi;
-  v[i] = vi;
-  w[i] -= lr * (mi / b1c) / (sqrtf(vi / b2c) + eps);
 }
 
 // inference fragments from the masters
@@ -603,7 +675,7 @@ struct SelectorState {
   int* log_count = nullptr;    // device counter
   // training scratch
   DevBuf scratch;
-  int scratch_B = 0;
+  int scratch_B = 0, scratch_rows = 0;
   // inference scratch for host-buffer calls
   DevBuf io, xio;
 };
@@ -780,15 +852,22 @@ void selector_log_buffers(const wsbb_ctx* ctx, float** feat, int** label, int** 
 
 static size_t wgrad_part_floats(const SelectorState* S, int B) {
   const size_t splits = (static_cast<size_t>(B) + kWgradK - 1) / kWgradK;
-  return splits * std::max(static_cast<size_t>(kHidden + 1) * S->P, static_cast<size_t>(S->F + 1) * kHidden);
+  return splits * (static_cast<size_t>(kHidden + 1) * S->P + static_cast<size_t>(S->F + 1) * kHidden);
 }
 
-static hipError_t ensure_scratch(SelectorState* S, int B) {
-  if (S->scratch_B >= B) return hipSuccess;
-  const size_t bytes = sizeof(float) * (static_cast<size_t>(B) * (S->F + 3 * kHidden + 2 * S->P + 1)) +
-                       sizeof(int) * B + 1024 + sizeof(float) * wgrad_part_floats(S, B) + 256;
+// training scratch for minibatches of B rows out of `rows` (an epoch's row
+// order and losses stay on the device)
+static hipError_t ensure_scratch(SelectorState* S, int B, int rows) {
+  if (S->scratch_B >= B && S->scratch_rows >= rows) return hipSuccess;
+  B = std::max(B, S->scratch_B);
+  rows = std::max(rows, S->scratch_rows);
+  const size_t bytes =
+      sizeof(float) * (static_cast<size_t>(B) * (S->F + 2 * kHidden + S->P) +
+                       static_cast<size_t>(kHidden) * (S->F + 2 * S->P) + wgrad_part_floats(S, B)) +
+      (sizeof(float) + sizeof(int)) * static_cast<size_t>(rows) + 512;
   hipError_t e = S->scratch.reserve(bytes);
-  if (e == hipSuccess) S->scratch_B = B;
+  S->scratch_B = e == hipSuccess ? B : 0;
+  S->scratch_rows = e == hipSuccess ? rows : 0;
   return e;
 }
 
@@ -800,53 +879,42 @@ static TrainArgs train_args(SelectorState* S, int B) {
   T.feat = S->log_feat;
   T.ldf = S->log_cap;
   T.label = S->log_label;
-  T.W1 = S->W1;
   T.b1 = S->b1;
-  T.W2 = S->W2;
   T.b2 = S->b2;
   float* p = S->scratch.as<float>();
-  T.X = p;
-  p += static_cast<size_t>(B) * S->F;
-  T.A1 = p;
-  p += static_cast<size_t>(B) * kHidden;
-  T.Hb = p;
-  p += static_cast<size_t>(B) * kHidden;
-  T.Z = p;
-  p += static_cast<size_t>(B) * S->P;
-  T.dZ = p;
-  p += static_cast<size_t>(B) * S->P;
-  T.dH = p;
-  p += static_cast<size_t>(B) * kHidden;
-  T.loss = p;
-  p += B;
+  auto take = [&](size_t n) {
+    float* q = p;
+    p += n;
+    return q;
+  };
+  const size_t cap = S->scratch_B;
+  T.X = take(cap * S->F);
+  T.Hb = take(cap * kHidden);
+  T.dZ = take(cap * S->P);
+  T.dH = take(cap * kHidden);
+  T.W1r = take(static_cast<size_t>(S->F) * kHidden);
+  T.W2r = take(static_cast<size_t>(kHidden) * S->P);
+  T.W2t = take(static_cast<size_t>(kHidden) * S->P);
+  T.part = take(wgrad_part_floats(S, S->scratch_B));
+  T.loss = take(S->scratch_rows);
   T.idx = reinterpret_cast<int*>(p);
-  T.part = reinterpret_cast<float*>(reinterpret_cast<uintptr_t>(T.idx + B + 64) & ~uintptr_t(255));
-  T.gW1 = S->gW1;
-  T.gb1 = S->gb1;
-  T.gW2 = S->gW2;
-  T.gb2 = S->gb2;
   return T;
 }
 
+// the weights rounded for the products, from the masters
+static void launch_round(wsbb_ctx* ctx, const TrainArgs& T) {
+  const int np = param_count(*ctx->selector);
+  hipLaunchKernelGGL(k_tr_round, dim3((np + 255) / 256), dim3(256), 0, ctx->stream, T,
+                     ctx->selector->W1, np);
+}
+
+// forward and backward of rows idx[0..B): partial weight gradients in part
 static void launch_fwd_bwd(wsbb_ctx* ctx, const TrainArgs& T) {
-  hipStream_t st = ctx->stream;
-  auto g = [](long long n) { return dim3(static_cast<unsigned>((n + 255) / 256)); };
-  hipLaunchKernelGGL(k_tr_in, g(1LL * T.B * T.F), dim3(256), 0, st, T);
-  hipLaunchKernelGGL(k_tr_hidden, g(1LL * T.B * kHidden), dim3(256), 0, st, T);
-  hipLaunchKernelGGL(k_tr_out, g(1LL * T.B * T.P), dim3(256), 0, st, T);
-  hipLaunchKernelGGL(k_tr_softmax, dim3((T.B + 3) / 4), dim3(256), 0, st, T);
-  const int splits = (T.B + kWgradK - 1) / kWgradK;
-  // gW2 = Hb^T dZ, gb2 = column sums of dZ
-  hipLaunchKernelGGL(k_tr_wgrad, dim3((kHidden + 1 + 63) / 64, (T.P + 63) / 64, splits), dim3(256), 0,
-                     st, T.Hb, kHidden, T.dZ, T.P, T.B, T.part);
-  hipLaunchKernelGGL(k_tr_wreduce, g(1LL * (kHidden + 1) * T.P), dim3(256), 0, st, T.part, kHidden,
-                     T.P, splits, T.gW2, T.gb2);
-  hipLaunchKernelGGL(k_tr_dH, g(1LL * T.B * kHidden), dim3(256), 0, st, T);
-  // gW1 = X^T dH, gb1 = column sums of dH
-  hipLaunchKernelGGL(k_tr_wgrad, dim3((T.F + 1 + 63) / 64, (kHidden + 63) / 64, splits), dim3(256), 0,
-                     st, T.X, T.F, T.dH, kHidden, T.B, T.part);
-  hipLaunchKernelGGL(k_tr_wreduce, g(1LL * (T.F + 1) * kHidden), dim3(256), 0, st, T.part, T.F,
-                     kHidden, splits, T.gW1, T.gb1);
+  hipLaunchKernelGGL(k_tr_rows, dim3((T.B + kTrainRows - 1) / kTrainRows), dim3(kTrainThreads), 0,
+                     ctx->stream, T);
+  hipLaunchKernelGGL(k_tr_wgrad,
+                     dim3(wgrad_tiles(kHidden, T.P) + wgrad_tiles(T.F, kHidden), (T.B + kWgradK - 1) / kWgradK),
+                     dim3(256), 0, ctx->stream, T);
 }
 
 }  // namespace wsbb
@@ -1011,11 +1079,15 @@ int wsbb_selector_grad(wsbb_ctx* ctx, const int32_t* idx, int B, float* loss, fl
     }
     nvalid += lab[idx[b]] >= 0;
   }
-  SEL_HIP(ensure_scratch(S, B), "hipMalloc(train scratch)");
+  SEL_HIP(ensure_scratch(S, B, B), "hipMalloc(train scratch)");
   TrainArgs T = train_args(S, B);
   T.nvalid = std::max(nvalid, 1);
   SEL_HIP(hipMemcpyAsync(const_cast<int*>(T.idx), idx, sizeof(int) * B, hipMemcpyHostToDevice, ctx->stream), "H2D idx");
+  launch_round(ctx, T);
   launch_fwd_bwd(ctx, T);
+  const int np = param_count(*S);
+  hipLaunchKernelGGL(k_tr_update<false>, dim3((np + 255) / 256), dim3(256), 0, ctx->stream, T, S->W1,
+                     S->mW1, S->vW1, S->gW1, np, (B + kWgradK - 1) / kWgradK, 0.f, 1.f, 1.f);
   SEL_HIP(hipGetLastError(), "train launch");
   std::vector<float> l(B);
   SEL_HIP(hipMemcpyAsync(l.data(), T.loss, sizeof(float) * B, hipMemcpyDeviceToHost, ctx->stream), "D2H loss");
@@ -1051,33 +1123,37 @@ int wsbb_selector_train(wsbb_ctx* ctx, int epochs, int batch, float lr, uint64_t
     return WSBB_EINVAL;
   }
   batch = std::min<int>(batch, static_cast<int>(rows.size()));
-  SEL_HIP(ensure_scratch(S, batch), "hipMalloc(train scratch)");
-  TrainArgs T = train_args(S, batch);
-  T.nvalid = batch;
+  const int nrows = static_cast<int>(rows.size()), nb = nrows / batch, used = nb * batch;
+  SEL_HIP(ensure_scratch(S, batch, nrows), "hipMalloc(train scratch)");
+  const TrainArgs T0 = train_args(S, batch);
   std::mt19937_64 rng(seed);
-  const int np = param_count(*S);
-  std::vector<float> lbuf(batch);
+  const int np = param_count(*S), splits = (batch + kWgradK - 1) / kWgradK;
+  std::vector<float> lbuf(used);
+  launch_round(ctx, T0);
   for (int ep = 0; ep < epochs; ++ep) {
     std::shuffle(rows.begin(), rows.end(), rng);
-    double tot = 0;
-    int nb = 0;
-    for (size_t start = 0; start + batch <= rows.size(); start += batch) {
-      SEL_HIP(hipMemcpyAsync(const_cast<int*>(T.idx), rows.data() + start, sizeof(int) * batch,
-                             hipMemcpyHostToDevice, ctx->stream),
-              "H2D idx");
+    // the epoch's row order goes up and its losses come back in one copy each
+    SEL_HIP(hipMemcpyAsync(const_cast<int*>(T0.idx), rows.data(), sizeof(int) * used,
+                           hipMemcpyHostToDevice, ctx->stream),
+            "H2D idx");
+    for (int i = 0; i < nb; ++i) {
+      TrainArgs T = T0;
+      T.idx += static_cast<size_t>(i) * batch;
+      T.loss += static_cast<size_t>(i) * batch;
+      T.nvalid = batch;
       launch_fwd_bwd(ctx, T);
       ++S->adam_t;
       const float b1c = 1.f - std::pow(0.9f, static_cast<float>(S->adam_t));
       const float b2c = 1.f - std::pow(0.999f, static_cast<float>(S->adam_t));
-      hipLaunchKernelGGL(k_adam, dim3((np + 255) / 256), dim3(256), 0, ctx->stream, S->W1, S->mW1,
-                         S->vW1, S->gW1, np, lr, b1c, b2c);
-      SEL_HIP(hipGetLastError(), "train launch");
-      SEL_HIP(hipMemcpyAsync(lbuf.data(), T.loss, sizeof(float) * batch, hipMemcpyDeviceToHost, ctx->stream),
-              "D2H loss");
-      SEL_HIP(hipStreamSynchronize(ctx->stream), "sync");
-      for (float x : lbuf) tot += x;
-      ++nb;
+      hipLaunchKernelGGL(k_tr_update<true>, dim3((np + 255) / 256), dim3(256), 0, ctx->stream, T,
+                         S->W1, S->mW1, S->vW1, S->gW1, np, splits, lr, b1c, b2c);
     }
+    SEL_HIP(hipGetLastError(), "train launch");
+    SEL_HIP(hipMemcpyAsync(lbuf.data(), T0.loss, sizeof(float) * used, hipMemcpyDeviceToHost, ctx->stream),
+            "D2H loss");
+    SEL_HIP(hipStreamSynchronize(ctx->stream), "sync");
+    double tot = 0;
+    for (float x : lbuf) tot += x;
     if (epoch_loss) epoch_loss[ep] = nb ? static_cast<float>(tot / nb) : 0.f;
   }
   S->frags_fresh = false;
