@@ -111,3 +111,35 @@ def test_mixed_batch_learned_is_a_valid_bound():
     assert (sub <= full).all()
     assert np.array_equal(fb, full)
     assert st["pairs"] < len(full) * 190
+
+
+@pytest.mark.parametrize("sizes,counts", [
+    # one class (equal padded sizes), uneven counts with an empty instance
+    ([(20, 5), (18, 6), (20, 8)], [1, 0, 333]),
+    # a class per instance, one node more and less than a block
+    ([(20, 20), (50, 20), (33, 9), (65, 5), (100, 10)], [257, 255, 129, 127, 64]),
+    # an instance beyond the matrix-core form: every instance runs the scan
+    ([(20, 5), (127, 4)], [70, 70])])
+def test_plain_batches_by_class(sizes, counts):
+    rng = np.random.default_rng(len(sizes))
+    ps = [rng.integers(1, 100, size=(m, n)).astype(np.int32) for n, m in sizes]
+    maxn, N = max(n for n, _ in sizes), sum(counts)
+    permT = np.zeros((maxn, N), np.uint8)
+    l1, l2 = np.zeros(N, np.int32), np.zeros(N, np.int32)
+    off = np.r_[0, np.cumsum(counts)].astype(np.int32)
+    ref = np.zeros(N, np.int32)
+    for i, p in enumerate(ps):
+        at, n = slice(off[i], off[i + 1]), p.shape[1]
+        if counts[i] == 0:
+            continue
+        permT[:n, at], l1[at], l2[at] = oracle.random_nodes(n, counts[i], 100 + i)
+        ref[at] = oracle.Oracle(p).bound_batch(np.ascontiguousarray(permT[:n, at]), l1[at], l2[at],
+                                               threads=8)
+    with wsbb_amd.Multi(ps) as mb:
+        mb.load(permT, l1, l2, off)
+        for reps in (1, 2):
+            got, st, _ = mb.run(reps=reps)
+            assert np.array_equal(got, ref)
+            assert st["nodes"] == N * reps and st["fallbacks"] == 0
+            assert st["pairs"] == reps * sum(c * p.shape[0] * (p.shape[0] - 1) // 2
+                                             for c, p in zip(counts, ps))

@@ -283,7 +283,10 @@ int wsbb_create(const int32_t* p, int n, int m, int device, wsbb_ctx** out) {
   const size_t o_Q0 = o_R0 + 256;
   const size_t o_tot = o_Q0 + 256;
   const size_t total = o_tot + 256;
-  if ((e = ctx->tables.reserve(total)) != hipSuccess) return fail(e, "hipMalloc(tables)");
+  // the matrix-core operands follow, built on the device (johnson.hip)
+  const size_t o_mf = total, b_mf = johnson_bytes(n, m), b_pf = johnson_time_bytes(n);
+  const size_t b_frag = johnson_fits(I) ? b_mf + b_pf + 32 * size_t(n) : 0;
+  if ((e = ctx->tables.reserve(total + b_frag)) != hipSuccess) return fail(e, "hipMalloc(tables)");
   std::vector<char> blob(total, 0);
   std::memcpy(blob.data() + o_steps, steps.data(), steps.size() * sizeof(int4));
   std::memcpy(blob.data() + o_wsel, wsel.data(), wsel.size() * sizeof(uint2));
@@ -311,18 +314,15 @@ int wsbb_create(const int32_t* p, int n, int m, int device, wsbb_ctx** out) {
   T.Q0 = ctx->tables.as<const int32_t>(o_Q0);
   T.ptot = ctx->tables.as<const int32_t>(o_tot);
   T.steps16 = two16 ? ctx->tables.as<const uint2>(o_s16) : nullptr;
-  if (johnson_fits(I)) {
-    const size_t b_mf = johnson_bytes(n, m), b_pf = johnson_time_bytes(n);
-    if ((e = ctx->frags.reserve(b_mf + b_pf + 32 * size_t(n))) != hipSuccess) return fail(e, "hipMalloc(fragments)");
-    T.mf = ctx->frags.as<const int4>();
-    T.pf = ctx->frags.as<const int4>(b_mf);
-    T.pr = ctx->frags.as<const int4>(b_mf + b_pf);
-    if ((e = build_johnson(T, ctx->frags.as<int4>(), ctx->frags.as<int4>(b_mf),
-                           ctx->frags.as<int4>(b_mf + b_pf), ctx->stream)) != hipSuccess)
+  if (b_frag > 0) {
+    T.mf = ctx->tables.as<const int4>(o_mf);
+    T.pf = ctx->tables.as<const int4>(o_mf + b_mf);
+    T.pr = ctx->tables.as<const int4>(o_mf + b_mf + b_pf);
+    // in order on the context's stream; whoever reads the tables on another
+    // one waits for it first
+    if ((e = build_johnson(T, ctx->tables.as<int4>(o_mf), ctx->tables.as<int4>(o_mf + b_mf),
+                           ctx->tables.as<int4>(o_mf + b_mf + b_pf), ctx->stream)) != hipSuccess)
       return fail(e, "fragment kernel launch");
-    // the tables are complete before any stream reads them (a mixed batch
-    // reads every instance's on one)
-    if ((e = hipStreamSynchronize(ctx->stream)) != hipSuccess) return fail(e, "hipStreamSynchronize");
   }
   *out = ctx;
   return WSBB_OK;
@@ -335,7 +335,6 @@ int wsbb_destroy(wsbb_ctx* ctx) {
   destroy_search(ctx);
   destroy_selector(ctx);
   ctx->tables.release();
-  ctx->frags.release();
   ctx->batch.release();
   if (ctx->ev_start) (void)hipEventDestroy(ctx->ev_start);
   if (ctx->ev_stop) (void)hipEventDestroy(ctx->ev_stop);

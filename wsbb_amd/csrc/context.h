@@ -61,7 +61,6 @@ struct wsbb_ctx {
   wsbb::Instance inst;
   wsbb::DevTables T{};
   wsbb::DevBuf tables;  // every instance table in one allocation
-  wsbb::DevBuf frags;   // matrix-core operands of the instance (johnson.hip)
   wsbb::DevBuf batch;   // staging for host-buffer batch calls
   wsbb::Launch launch;
   int pool_capacity = 1 << 24;  // device node-pool capacity (nodes)

@@ -194,6 +194,29 @@ struct Child {
   bool two;
 };
 
+// one of an array of tables, word by word through scalar loads (i uniform)
+__device__ __forceinline__ DevTables tables_at(const DevTables* tabs, int i) {
+  static_assert(sizeof(DevTables) % 4 == 0, "word copy");
+  DevTables T;
+  const int* src = reinterpret_cast<const int*>(tabs + i);
+  int* dst = reinterpret_cast<int*>(&T);
+#pragma unroll
+  for (int k = 0; k < static_cast<int>(sizeof(DevTables) / 4); ++k) dst[k] = ld_const(src, k);
+  return T;
+}
+
+// Node source: explicit nodes of several instances, each block's of one.
+struct MultiSource {
+  static constexpr bool kState = false;
+  const DevTables* tabs;  // [instances]
+  const int4* blocks;     // {instance, first node, node count, 0}
+  BatchSource nodes;      // all instances' nodes, [max n][N]
+  __device__ __forceinline__ bool load(int k, int& a, int& b, const uint8_t*& col,
+                                       int& stride, int& sw0, int& sw1) const {
+    return nodes.load(k, a, b, col, stride, sw0, sw1);
+  }
+};
+
 // Node source: children described by (parent, side, position) over a
 // position-major parent array (decompose_beginend child semantics).
 struct ChildSource {

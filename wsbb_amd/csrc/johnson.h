@@ -8,6 +8,10 @@ namespace wsbb {
 
 // x_k = lag + p_a is split as lo + kXBase hi, both in a signed byte
 constexpr int kXBase = 127;
+// 32-wide column blocks of n jobs and the two constants
+__host__ __device__ inline int column_blocks(int n) { return (n + 33) >> 5; }
+// register arrays over machines: 8, 12, 16, 20 or 24
+inline int padded_machines(int m) { return m <= 8 ? 8 : (m + 3) & ~3; }
 constexpr int kXMax = kXBase * kXBase + kXBase - 1;
 
 // Couples of pairs of m machines (k_johnson walks two pairs of one first
@@ -24,9 +28,9 @@ __host__ __device__ inline int johnson_couples(int m) { return johnson_first_cou
 // couple, and its bytes: one KiB per entry, 32 rows and 32 columns.
 __host__ __device__ inline int johnson_entries(int m) { return 2 * (johnson_couples(m) + 4); }
 inline size_t johnson_bytes(int n, int m) {
-  return static_cast<size_t>(johnson_entries(m)) * ((n + 31) >> 5) * ((n + 33) >> 5) * 1024;
+  return static_cast<size_t>(johnson_entries(m)) * ((n + 31) >> 5) * column_blocks(n) * 1024;
 }
-inline size_t johnson_time_bytes(int n) { return static_cast<size_t>((n + 33) >> 5) * 1024; }
+inline size_t johnson_time_bytes(int n) { return static_cast<size_t>(column_blocks(n)) * 1024; }
 
 // How a launch is laid out over waves and LDS (set by the launcher).
 struct JohnsonShape {
@@ -36,8 +40,16 @@ struct JohnsonShape {
   int tile_bytes;  // LDS of one tile
   int first_block; // of this launch
   int list_rows;   // 64-word rows of a tile's pair list
+  int wide;        // tiles of 128 nodes, not 64
   const int* list; // the children to bound, or null: all of them
 };
+
+// The layout for N nodes; waves: ways to split the pairs, or 0 (chosen).
+JohnsonShape johnson_shape(int n, int P, int N, int waves, bool subset, int num_cus);
+inline int johnson_block_nodes(const JohnsonShape& H) { return (H.wide ? 128 : 64) * H.tpb; }
+// Instances of one class share a kernel: equal padded machines, row tiles and
+// column blocks.
+int johnson_class(int n, int m);
 
 // Fills mf (johnson_bytes), pf (johnson_time_bytes) and pr (32 n bytes) from
 // T's step table and times.
@@ -48,6 +60,10 @@ hipError_t build_johnson(const DevTables& T, int4* mf, int4* pf, int4* pr, hipSt
 hipError_t launch_johnson(const DevTables& T, const BatchSource& src, const BoundArgs& A,
                           int grid_cap, hipStream_t stream);
 hipError_t launch_johnson(const DevTables& T, const ChildSource& src, const BoundArgs& A,
+                          int grid_cap, hipStream_t stream);
+// Nodes of several instances of one class; T: the class's largest n and P, A.N
+// its nodes; every block holds at most johnson_block_nodes of one instance.
+hipError_t launch_johnson(const DevTables& T, const MultiSource& src, const BoundArgs& A, int blocks,
                           int grid_cap, hipStream_t stream);
 hipError_t launch_johnson(const DevTables& T, const ListSource& src, const BoundArgs& A,
                           int grid_cap, hipStream_t stream);

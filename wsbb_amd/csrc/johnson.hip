@@ -93,7 +93,7 @@ __global__ __launch_bounds__(256) void k_johnson_tables(DevTables T, int4* mf, i
     b = min(b + (at_s & 1), m - 1);
     s = a * m - a * (a + 1) / 2 + b - a - 1;
   }
-  const int rts = (n + 31) >> 5, kbs = (n + 33) >> 5;
+  const int rts = (n + 31) >> 5, kbs = column_blocks(n);
   const RowMap rm(n, rts);
   if (at_s < 0) {
     for (int u = threadIdx.x; u < kbs * 64; u += blockDim.x) {
@@ -220,13 +220,26 @@ struct Layout {
 //
 // SUBSET: each tile (of 64 nodes) walks its own pairs.
 template <int MM, int KB, int NR, int NB, bool SUBSET, class Src>
-__global__ __launch_bounds__(256, (NB == 2 && KB <= 2 ? 3 : 2)) void k_johnson(DevTables T, Src src,
+__global__ __launch_bounds__(256, (NB == 2 && KB <= 2 ? 3 : 2)) void k_johnson(DevTables T0, Src src,
                                                                               BoundArgs A,
                                                                               JohnsonShape H) {
   extern __shared__ char lds[];
   constexpr int rs = row_bytes(MM);
   constexpr int TN = 32 * NB;      // nodes of a tile
   constexpr int RUNS = NB / 2;     // runs of 64 nodes in a tile, each way
+  constexpr bool MULTI = std::is_same<Src, MultiSource>::value;
+  const int bt = H.first_block + blockIdx.x;
+  // the block's instance and nodes: all of the launch's, or its own
+  int first = bt * (TN * H.tpb), N = 0;
+  DevTables T = T0;
+  if constexpr (MULTI) {
+    const int* b = reinterpret_cast<const int*>(src.blocks + bt);
+    T = tables_at(src.tabs, ld_const(b, 0));
+    first = ld_const(b, 1);
+    N = first + ld_const(b, 2);
+  } else {
+    N = (A.Ndev != nullptr) ? *A.Ndev : A.N;
+  }
   const int n = T.n, m = T.m;
   const int rts = H.rts, G = H.groups, W = rts * G;
   const int waves = blockDim.x >> 6;
@@ -246,9 +259,7 @@ __global__ __launch_bounds__(256, (NB == 2 && KB <= 2 ? 3 : 2)) void k_johnson(D
   uint16_t* order = lens + nodes;                                  // [2][nodes]
   uint8_t* rows = reinterpret_cast<uint8_t*>(lds + L.rows);        // [n][rs]
 
-  const int N = (A.Ndev != nullptr) ? *A.Ndev : A.N;
-  const int bt = H.first_block + blockIdx.x;
-  const int node0 = bt * nodes;              // the block's first node
+  const int node0 = first;                   // the block's first node
   const int tile0 = node0 + tib * TN;        // this wave's tile's
   // a child's descriptor is read at any index below the capacity while the
   // live count is on its way; past the count it is read again in range
@@ -736,16 +747,14 @@ __global__ __launch_bounds__(256, (NB == 2 && KB <= 2 ? 3 : 2)) void k_johnson(D
 
 template <int MM, int KB, int NR, int NB, bool SUBSET, class Src>
 hipError_t launch_kernel(const DevTables& T, const Src& src, const BoundArgs& A, JohnsonShape H,
-                         int grid_cap, hipStream_t stream) {
+                         int blocks, int grid_cap, hipStream_t stream) {
   constexpr int rs = row_bytes(MM), TN = 32 * NB;
   const int waves = H.rts * H.groups * H.tpb;
   const int body = std::max(Src::kState ? 0 : T.n * TN, 2 * MM * TN * 4);
   H.tile_bytes = ((body + 15) & ~15) + 2 * H.rts * TN * 4;
-  const int nodes = TN * H.tpb;
   H.list_rows = (T.P + 63) / 64;
-  const size_t shmem = Layout(H.tpb, H.tile_bytes, waves, nodes, T.n, rs).total +
+  const size_t shmem = Layout(H.tpb, H.tile_bytes, waves, TN * H.tpb, T.n, rs).total +
                        (SUBSET ? 256 * H.list_rows * H.tpb : 0);
-  const int blocks = (A.N + nodes - 1) / nodes;
   // a block bounds its tiles and ends (a loop over tiles kept the whole
   // prologue's constants in registers); more blocks than the cap run as
   // several launches
@@ -760,70 +769,52 @@ hipError_t launch_kernel(const DevTables& T, const Src& src, const BoundArgs& A,
   return hipSuccess;
 }
 
+// `blocks` > 0: the length of a MultiSource's list
 template <int MM, class Src>
-hipError_t launch_mm(const DevTables& T, const Src& src, const BoundArgs& A, const int* list,
-                     int grid_cap, hipStream_t stream) {
+hipError_t launch_mm(const DevTables& T, const Src& src, const BoundArgs& A, JohnsonShape H,
+                     int blocks, int grid_cap, hipStream_t stream) {
   const bool subset = A.tile_sel != nullptr;
-  const int kb = (T.n + 33) >> 5;
-  JohnsonShape H{};
-  H.list = list;
-  H.rts = (T.n + 31) >> 5;
-  const int simds = 4 * A.num_cus, tiles = (A.N + 63) / 64;
-  // The pairs are split over waves while that still adds waves to SIMDs that
-  // have few, and where a tile's pairs outweigh the heads and tails that the
-  // split leaves to one wave (us at G = 1 / 2 / 4: 20x20, 50 000 nodes 34 / 27
-  // / 25; 100 003 nodes 41 / 37 / 43; 300 000 nodes 83 / 85 / 109; 30x12,
-  // 100 000 nodes 24 / 28 / 34).
-  H.groups = A.waves > 0                               ? A.waves
-             : tiles * H.rts < simds                   ? 4
-             : tiles * H.rts < 2 * simds && T.P >= 128 ? 2
-                                                       : 1;
-  H.groups = subset ? 1 : std::max(1, std::min(H.groups, 4 / H.rts));
-  // Tiles of 128 nodes halve the fragments' way through the L1 and the scalar
-  // work, for twice the registers: with two column blocks of jobs and more,
-  // from two waves per SIMD on (us for 64 / 128 nodes: 50x20, 65 536 nodes 56
-  // / 66; 130 000 nodes 101 / 93; 2^20 nodes 654 / 600; 100x10, 65 521 nodes
-  // 70 / 55).  With one, the start clocks and tails of 128 nodes leave room
-  // in LDS for one wave per SIMD (20x20, 300 000 nodes: 83 / 151).
-  const bool wide = !subset && kb >= 2 && H.groups == 1 &&
-                    static_cast<long long>((A.N + 127) / 128) * H.rts >= 2 * simds;
-  H.tpb = std::max(1, 4 / (H.rts * H.groups));
-  const int per = RowMap(T.n, H.rts).per;
+  if (blocks == 0) {
+    const int nodes = johnson_block_nodes(H);
+    blocks = (A.N + nodes - 1) / nodes;
+  }
   using std::integral_constant;
   auto rows = [&](auto kbv, auto nrv) {
     constexpr int KB = decltype(kbv)::value, NR = decltype(nrv)::value;
     if constexpr (std::is_same<Src, ChildSource>::value)
-      if (subset) return launch_kernel<MM, KB, NR, 2, true, Src>(T, src, A, H, grid_cap, stream);
+      if (subset)
+        return launch_kernel<MM, KB, NR, 2, true, Src>(T, src, A, H, blocks, grid_cap, stream);
     if constexpr (KB >= 2)
-      if (wide) return launch_kernel<MM, KB, NR, 4, false, Src>(T, src, A, H, grid_cap, stream);
-    return launch_kernel<MM, KB, NR, 2, false, Src>(T, src, A, H, grid_cap, stream);
+      if (H.wide)
+        return launch_kernel<MM, KB, NR, 4, false, Src>(T, src, A, H, blocks, grid_cap, stream);
+    return launch_kernel<MM, KB, NR, 2, false, Src>(T, src, A, H, blocks, grid_cap, stream);
   };
-  auto blocks = [&](auto kbv) {
-    constexpr int KB = decltype(kbv)::value;
-    if constexpr (KB == 1) {
-      if (per <= 10) return rows(kbv, integral_constant<int, 10>{});
-    } else {
-      if (per <= 13) return rows(kbv, integral_constant<int, 13>{});
-    }
-    return rows(kbv, integral_constant<int, 16>{});
+  const bool few = RowMap(T.n, H.rts).per <= (column_blocks(T.n) == 1 ? 10 : 13);
+  auto pick = [&](auto kbv) {
+    constexpr int FEW = decltype(kbv)::value == 1 ? 10 : 13;
+    return few ? rows(kbv, integral_constant<int, FEW>{}) : rows(kbv, integral_constant<int, 16>{});
   };
-  switch (kb) {
-    case 1: return blocks(integral_constant<int, 1>{});
-    case 2: return blocks(integral_constant<int, 2>{});
-    case 3: return blocks(integral_constant<int, 3>{});
-    case 4: return blocks(integral_constant<int, 4>{});
+  switch (column_blocks(T.n)) {
+    case 1: return pick(integral_constant<int, 1>{});
+    case 2: return pick(integral_constant<int, 2>{});
+    case 3: return pick(integral_constant<int, 3>{});
+    case 4: return pick(integral_constant<int, 4>{});
     default: return hipErrorInvalidValue;
   }
 }
 
 template <class Src>
 hipError_t launch_src(const DevTables& T, const Src& src, const BoundArgs& A, const int* list,
-                      int grid_cap, hipStream_t stream) {
-  if (T.m <= 8) return launch_mm<8>(T, src, A, list, grid_cap, stream);
-  if (T.m <= 12) return launch_mm<12>(T, src, A, list, grid_cap, stream);
-  if (T.m <= 16) return launch_mm<16>(T, src, A, list, grid_cap, stream);
-  if (T.m <= 20) return launch_mm<20>(T, src, A, list, grid_cap, stream);
-  return launch_mm<24>(T, src, A, list, grid_cap, stream);
+                      int blocks, int grid_cap, hipStream_t stream) {
+  JohnsonShape H = johnson_shape(T.n, T.P, A.N, A.waves, A.tile_sel != nullptr, A.num_cus);
+  H.list = list;
+  switch (padded_machines(T.m)) {
+    case 8: return launch_mm<8>(T, src, A, H, blocks, grid_cap, stream);
+    case 12: return launch_mm<12>(T, src, A, H, blocks, grid_cap, stream);
+    case 16: return launch_mm<16>(T, src, A, H, blocks, grid_cap, stream);
+    case 20: return launch_mm<20>(T, src, A, H, blocks, grid_cap, stream);
+    default: return launch_mm<24>(T, src, A, H, blocks, grid_cap, stream);
+  }
 }
 
 }  // namespace
@@ -833,19 +824,57 @@ hipError_t build_johnson(const DevTables& T, int4* mf, int4* pf, int4* pr, hipSt
   return hipGetLastError();
 }
 
+JohnsonShape johnson_shape(int n, int P, int N, int waves, bool subset, int num_cus) {
+  JohnsonShape H{};
+  H.rts = (n + 31) >> 5;
+  const int simds = 4 * num_cus, tiles = (N + 63) / 64;
+  // The pairs are split over waves while that still adds waves to SIMDs that
+  // have few, and where a tile's pairs outweigh the heads and tails that the
+  // split leaves to one wave (us at G = 1 / 2 / 4: 20x20, 50 000 nodes 34 / 27
+  // / 25; 100 003 nodes 41 / 37 / 43; 300 000 nodes 83 / 85 / 109; 30x12,
+  // 100 000 nodes 24 / 28 / 34).
+  H.groups = waves > 0                               ? waves
+             : tiles * H.rts < simds                 ? 4
+             : tiles * H.rts < 2 * simds && P >= 128 ? 2
+                                                     : 1;
+  H.groups = subset ? 1 : std::max(1, std::min(H.groups, 4 / H.rts));
+  // Tiles of 128 nodes halve the fragments' way through the L1 and the scalar
+  // work, for twice the registers: with two column blocks of jobs and more,
+  // from two waves per SIMD on (us for 64 / 128 nodes: 50x20, 65 536 nodes 56
+  // / 66; 130 000 nodes 101 / 93; 2^20 nodes 654 / 600; 100x10, 65 521 nodes
+  // 70 / 55).  With one, the start clocks and tails of 128 nodes leave room
+  // in LDS for one wave per SIMD (20x20, 300 000 nodes: 83 / 151).
+  H.wide = !subset && column_blocks(n) >= 2 && H.groups == 1 &&
+           static_cast<long long>((N + 127) / 128) * H.rts >= 2 * simds;
+  H.tpb = std::max(1, 4 / (H.rts * H.groups));
+  return H;
+}
+
+int johnson_class(int n, int m) {
+  const int rts = (n + 31) >> 5, kb = column_blocks(n);
+  const bool few = RowMap(n, rts).per <= (kb == 1 ? 10 : 13);
+  return ((padded_machines(m) * 8 + rts) * 8 + kb) * 2 + few;
+}
+
+hipError_t launch_johnson(const DevTables& T, const MultiSource& src, const BoundArgs& A, int blocks,
+                          int grid_cap, hipStream_t stream) {
+  if (A.tile_sel || blocks < 1) return hipErrorInvalidValue;
+  return launch_src(T, src, A, nullptr, blocks, grid_cap, stream);
+}
+
 hipError_t launch_johnson(const DevTables& T, const BatchSource& src, const BoundArgs& A,
                           int grid_cap, hipStream_t stream) {
   if (A.tile_sel) return hipErrorInvalidValue;
-  return launch_src(T, src, A, nullptr, grid_cap, stream);
+  return launch_src(T, src, A, nullptr, 0, grid_cap, stream);
 }
 hipError_t launch_johnson(const DevTables& T, const ChildSource& src, const BoundArgs& A,
                           int grid_cap, hipStream_t stream) {
-  return src.has_state() ? launch_src(T, src, A, nullptr, grid_cap, stream) : hipErrorInvalidValue;
+  return src.has_state() ? launch_src(T, src, A, nullptr, 0, grid_cap, stream) : hipErrorInvalidValue;
 }
 hipError_t launch_johnson(const DevTables& T, const ListSource& src, const BoundArgs& A,
                           int grid_cap, hipStream_t stream) {
   if (!src.has_state() || A.tile_sel) return hipErrorInvalidValue;
-  return launch_src(T, src.base, A, src.list, grid_cap, stream);
+  return launch_src(T, src.base, A, src.list, 0, grid_cap, stream);
 }
 
 }  // namespace wsbb

@@ -13,6 +13,12 @@
 // (full LB2).  Per node the result equals bound_flowshop::bornes_calculer
 // (src/bound_flowshop.cpp:929-951) of its own instance, or the LB2 over the
 // tile's subset.
+//
+// Plain LB2 of instances that fit the matrix-core form (johnson.hip) runs one
+// launch per class of sizes that share a kernel, each block on one instance's
+// nodes: 64 instances of nine sizes, 4099 nodes each, take 0.30 ms in nine
+// launches against 0.92 ms in the one launch of k_multi_bound, which keeps
+// learned subsets and instances beyond that form.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -23,6 +29,7 @@
 #include "../../include/wsbb_amd.h"
 #include "bound.h"
 #include "context.h"
+#include "johnson.h"
 #include "selector.h"
 
 struct wsbb_multi {
@@ -44,6 +51,15 @@ struct wsbb_multi {
   // per machine-count class: the tiles of its instances (in tile_list) and
   // the instance whose selector scores them
   std::vector<int> class_m, class_first, class_count, class_rep;
+  // plain LB2 on the matrix cores, one launch per class of instances that
+  // share a kernel (empty unless every instance fits): the class's sizes,
+  // nodes, and blocks in block_list
+  struct Johnson {
+    wsbb::DevTables T;
+    int nodes, first, blocks;
+  };
+  std::vector<Johnson> johnson;
+  int4* block_list = nullptr;  // {instance, first node, node count, 0}
   std::vector<int> offsets;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -69,17 +85,6 @@ struct MultiArgs {
   long long* stats;          // [3] nodes, fallbacks, node-pair evaluations
   float scale_unused;
 };
-
-// the tile's tables, word by word through scalar loads (inst is uniform)
-__device__ __forceinline__ DevTables tile_tables(const DevTables* tabs, int inst) {
-  static_assert(sizeof(DevTables) % 4 == 0, "word copy");
-  DevTables T;
-  const int* src = reinterpret_cast<const int*>(tabs + inst);
-  int* dst = reinterpret_cast<int*>(&T);
-#pragma unroll
-  for (int i = 0; i < static_cast<int>(sizeof(DevTables) / 4); ++i) dst[i] = ld_const(src, i);
-  return T;
-}
 
 // four Johnson steps, as in bound.hip
 __device__ __forceinline__ uint32_t bsel(uint32_t mask, uint32_t a, uint32_t b) {
@@ -133,7 +138,7 @@ __global__ __launch_bounds__(256) void k_multi_bound(MultiArgs A) {
   int staged = -1;
   for (int bt = blockIdx.x; bt < A.ntiles; bt += gridDim.x) {
     const int inst = __builtin_amdgcn_readfirstlane(A.tile_inst[bt]);
-    const DevTables T = tile_tables(A.tabs, inst);
+    const DevTables T = tables_at(A.tabs, inst);
     const int n = T.n, m = T.m, P = T.P;
     if (inst != staged) {
       __syncthreads();
@@ -287,7 +292,7 @@ __global__ __launch_bounds__(256) void k_multi_features(MultiFeatArgs A) {
     const int tile = __builtin_amdgcn_readfirstlane(t0 + wave);
     if (tile >= A.ntiles) continue;
     const int inst = __builtin_amdgcn_readfirstlane(A.tile_inst[tile]);
-    const DevTables T = tile_tables(A.tabs, inst);
+    const DevTables T = tables_at(A.tabs, inst);
     const int n = T.n, m = T.m;
     if (inst != staged) {
       for (int i = lane; i < MM * n; i += 64) sp[i] = i < m * n ? T.p[i] : 0;
@@ -421,6 +426,18 @@ namespace {
 
 int run_multi(wsbb_multi* M, int kind, int margin, bool have_tsel) {
   hipStream_t st = M->ctx[0]->stream;
+  if (kind != WSBB_LEARNED && !M->johnson.empty()) {
+    for (const auto& c : M->johnson) {
+      MultiSource src{M->tabs.as<const DevTables>(), M->block_list + c.first,
+                      BatchSource{M->permT, M->l1, M->l2, M->N}};
+      BoundArgs A{};
+      A.N = c.nodes;
+      A.num_cus = M->num_cus;
+      A.out = M->out;
+      MULTI_HIP(launch_johnson(c.T, src, A, c.blocks, 16 * M->num_cus, st), "multi bound launch");
+    }
+    return WSBB_OK;
+  }
   const int grid = std::max(1, std::min(M->ntiles, 8 * M->num_cus));
   if (kind == WSBB_LEARNED && !have_tsel) {
     MultiFeatArgs F{};
@@ -495,6 +512,13 @@ int wsbb_multi_create(int count, const int32_t* const* p, const int* n, const in
     M->nsw = std::max(M->nsw, (c->T.P + 31) / 32);
     M->fstride = std::max(M->fstride, (5 * m[i] + 7) / 8);
   }
+  // the batch runs on the first context's stream and reads every context's
+  // tables, which each context finishes on its own
+  for (wsbb_ctx* c : M->ctx)
+    if (hipError_t e = hipStreamSynchronize(c->stream); e != hipSuccess) {
+      wsbb_multi_destroy(M);
+      return hip_fail(e, "multi tables");
+    }
   M->num_cus = M->ctx[0]->num_cus;
   hipError_t e = M->tabs.reserve(sizeof(DevTables) * count);
   if (e == hipSuccess)
@@ -581,6 +605,34 @@ int wsbb_multi_load(wsbb_multi* M, const uint8_t* permT, const int32_t* l1, cons
       if (M->ctx[tinst[t]]->T.m == mi) tlist.push_back(t);
     M->class_count.push_back(static_cast<int>(tlist.size()) - M->class_first.back());
   }
+  // classes of instances that share a matrix-core kernel, and their blocks
+  std::vector<wsbb_multi::Johnson> johnson;
+  std::vector<int4> blocks;
+  bool fits = true;
+  for (const wsbb_ctx* c : M->ctx) fits = fits && c->T.mf != nullptr;
+  std::vector<int> cls(count), seen;
+  for (int i = 0; i < count; ++i) cls[i] = johnson_class(M->ctx[i]->T.n, M->ctx[i]->T.m);
+  for (int i = 0; fits && i < count; ++i) {
+    if (std::find(seen.begin(), seen.end(), cls[i]) != seen.end()) continue;
+    seen.push_back(cls[i]);
+    wsbb_multi::Johnson J{M->ctx[i]->T, 0, static_cast<int>(blocks.size()), 0};
+    for (int k = i; k < count; ++k)
+      if (cls[k] == cls[i]) {
+        const DevTables& T = M->ctx[k]->T;
+        J.nodes += offsets[k + 1] - offsets[k];
+        J.T.n = std::max(J.T.n, T.n);
+        J.T.m = std::max(J.T.m, T.m);
+        J.T.P = std::max(J.T.P, T.P);
+      }
+    if (J.nodes == 0) continue;
+    const int per = johnson_block_nodes(johnson_shape(J.T.n, J.T.P, J.nodes, 0, false, M->num_cus));
+    for (int k = i; k < count; ++k)
+      if (cls[k] == cls[i])
+        for (int at = offsets[k]; at < offsets[k + 1]; at += per)
+          blocks.push_back(int4{k, at, std::min(per, offsets[k + 1] - at), 0});
+    J.blocks = static_cast<int>(blocks.size()) - J.first;
+    johnson.push_back(J);
+  }
   std::vector<float> scale(count);
   for (int i = 0; i < count; ++i)
     scale[i] = static_cast<float>(M->ctx[i]->inst.path_bound > 0 ? M->ctx[i]->inst.path_bound : 1);
@@ -600,6 +652,7 @@ int wsbb_multi_load(wsbb_multi* M, const uint8_t* permT, const int32_t* l1, cons
   const size_t o_ts = take(4 * size_t(ntiles) * M->nsw);
   const size_t o_xf = take(sizeof(uint2) * 2 * size_t(ntiles) * M->fstride * 64);
   const size_t o_st = take(8 * 4);
+  const size_t o_bl = take(sizeof(int4) * std::max<size_t>(blocks.size(), 1));
   MULTI_HIP(hipSetDevice(M->device), "hipSetDevice");
   MULTI_HIP(M->batch.reserve(off), "hipMalloc(multi batch)");
   M->N = N;
@@ -616,6 +669,8 @@ int wsbb_multi_load(wsbb_multi* M, const uint8_t* permT, const int32_t* l1, cons
   M->tsel = M->batch.as<uint32_t>(o_ts);
   M->xfrag = M->batch.as<uint2>(o_xf);
   M->stats = M->batch.as<long long>(o_st);
+  M->block_list = M->batch.as<int4>(o_bl);
+  M->johnson = johnson;
   hipStream_t st = M->ctx[0]->stream;
   // rows past an instance's n are never read
   for (int r = 0; r < M->maxn; ++r)
@@ -627,6 +682,9 @@ int wsbb_multi_load(wsbb_multi* M, const uint8_t* permT, const int32_t* l1, cons
   MULTI_HIP(hipMemcpyAsync(M->tile_node0, tnode0.data(), 4 * size_t(ntiles), hipMemcpyHostToDevice, st), "H2D map");
   MULTI_HIP(hipMemcpyAsync(M->tile_cnt, tcnt.data(), 4 * size_t(ntiles), hipMemcpyHostToDevice, st), "H2D map");
   MULTI_HIP(hipMemcpyAsync(M->tile_list, tlist.data(), 4 * size_t(ntiles), hipMemcpyHostToDevice, st), "H2D list");
+  if (!blocks.empty())
+    MULTI_HIP(hipMemcpyAsync(M->block_list, blocks.data(), sizeof(int4) * blocks.size(),
+                             hipMemcpyHostToDevice, st), "H2D blocks");
   MULTI_HIP(hipMemcpyAsync(M->tile_list + ntiles, scale.data(), 4 * size_t(count), hipMemcpyHostToDevice, st),
             "H2D scales");
   M->offsets.assign(offsets, offsets + count + 1);
@@ -673,7 +731,13 @@ int wsbb_multi_run(wsbb_multi* M, int kind, const int32_t* inc, int margin,
     *ms = t / reps;
   }
   if (out) MULTI_HIP(hipMemcpy(out, M->out, 4 * size_t(M->N), hipMemcpyDeviceToHost), "D2H out");
-  if (stats) {
+  if (stats && kind != WSBB_LEARNED && !M->johnson.empty()) {
+    // every node over every pair of its instance
+    stats[0] = static_cast<int64_t>(M->N) * reps;
+    stats[1] = stats[2] = 0;
+    for (int i = 0; i < count; ++i)
+      stats[2] += static_cast<int64_t>(M->offsets[i + 1] - M->offsets[i]) * M->ctx[i]->T.P * reps;
+  } else if (stats) {
     long long h[3];
     MULTI_HIP(hipMemcpy(h, M->stats, sizeof(h), hipMemcpyDeviceToHost), "D2H stats");
     for (int i = 0; i < 3; ++i) stats[i] = h[i];
