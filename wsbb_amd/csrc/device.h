@@ -160,6 +160,32 @@ __device__ __forceinline__ void tail_step(int (&q)[MM], const int (&pk)[MM]) {
   for (int k = MM - 1; k >= 0; --k) q[k] = max(q[k], (k + 1 < MM) ? q[k + 1] : 0) + pk[k];
 }
 
+// Two jobs at once, first pa then pb: machine k of the first job and machine
+// k - 1 of the second do not depend on each other, so the chain of dependent
+// operations is half as long as two single steps'.
+template <int MM>
+__device__ __forceinline__ void head_step2(int (&r)[MM], const int (&pa)[MM], const int (&pb)[MM]) {
+  int a = r[0] + pa[0], b = 0;
+#pragma unroll
+  for (int k = 1; k <= MM; ++k) {
+    const int t = k < MM ? max(r[k], a) : 0, u = max(a, b);
+    b = u + pb[k - 1];
+    r[k - 1] = b;
+    if (k < MM) a = t + pa[k];
+  }
+}
+template <int MM>
+__device__ __forceinline__ void tail_step2(int (&q)[MM], const int (&pa)[MM], const int (&pb)[MM]) {
+  int a = q[MM - 1] + pa[MM - 1], b = 0;
+#pragma unroll
+  for (int k = MM - 2; k >= -1; --k) {
+    const int t = k >= 0 ? max(q[k], a) : 0, u = max(a, b);
+    b = u + pb[k + 1];
+    q[k + 1] = b;
+    if (k >= 0) a = t + pa[k];
+  }
+}
+
 __device__ __forceinline__ int perm_at(const uint8_t* col, int stride, int sw0,
                                        int sw1, int i) {
   const int src = (i == sw0) ? sw1 : ((i == sw1) ? sw0 : i);

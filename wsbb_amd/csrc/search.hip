@@ -638,29 +638,71 @@ __global__ __launch_bounds__(1024) void k_select_chain(SArgs S) {
 }
 
 // ---- expand: parents out of the stack, child descriptors ------------------
-// A thread per parent copies its permutation column (consecutive parents sit
-// at consecutive stack slots, so every position row is read coalesced),
-// writes its children's descriptors and computes the parent's heads, tails
-// and scheduled-job mask once: the bound kernel extends them by the one or
-// two jobs each child places instead of rerunning the recurrences over the
-// whole prefix and suffix per child.  Written for latency (a round has a few
-// thousand parents): one batch of loads per column chunk, no lane exchanges.
-// small blocks: a round's parents (a few thousand) spread over many CUs
-// instead of filling a few
-constexpr int kExpandBlock = 64;
+// 64 parents a block, two waves: consecutive parents sit at consecutive stack
+// slots, so every position row is read coalesced.  The first wave copies the
+// permutation columns, then runs the prefixes (heads); the second runs the
+// suffixes (tails); both write the children's descriptors, a parent's at a
+// time.  The bound kernels extend a parent's heads and tails by the one or
+// two jobs each child places instead of rerunning them per child.
+//
+// Written for latency: a round has a few thousand parents, the recurrences
+// are the longest chain (one wave ran prefix and suffix one after the other,
+// and a thread wrote its parent's descriptors into lines of its own: 20x10,
+// 2900 parents 8.7 us, 50x20, 830 parents 19.4 us; in two waves and two jobs
+// a step 7.2 and 13.5 us; at 20x20, 34K parents, 17.3 became 16.0 us).
+constexpr int kExpandParents = 64, kExpandBlock = 2 * kExpandParents;
 
+// one recurrence over `len` positions from `first`, `step` apart, two jobs at
+// a time; the scheduled jobs to sm and, if wanted, their times to wk
+template <int MM, int NW, class One, class Two>
+__device__ __forceinline__ void expand_run(const int32_t* sp, const uint8_t* col, int first, int step,
+                                           int len, bool work, uint32_t (&sm)[NW], int (&wk)[MM],
+                                           One one, Two two) {
+  const uint8_t* c = col + first * kExpandParents;
+  const int d = step * kExpandParents;
+  int ja = len > 0 ? c[0] : 0, jb = len > 1 ? c[d] : 0;
+  int i = 0;
+  for (; i + 1 < len; i += 2) {
+    const int j = ja, k = jb;
+    int pa[MM], pb[MM];
+    job_row<MM>(sp, j, pa);
+    job_row<MM>(sp, k, pb);
+    if (i + 2 < len) ja = c[(i + 2) * d];
+    if (i + 3 < len) jb = c[(i + 3) * d];
+    set_job_bit<NW>(sm, j);
+    set_job_bit<NW>(sm, k);
+    two(pa, pb);
+    if (work)
+#pragma unroll
+      for (int q = 0; q < MM; ++q) wk[q] += pa[q] + pb[q];
+  }
+  if (i < len) {
+    int pk[MM];
+    job_row<MM>(sp, ja, pk);
+    set_job_bit<NW>(sm, ja);
+    one(pk);
+    if (work)
+#pragma unroll
+      for (int q = 0; q < MM; ++q) wk[q] += pk[q];
+  }
+}
+
+// want_state: 0 none, 1 heads, tails and scheduled jobs, 2 also their work
 template <int MM, int NW, bool FEAT>
 __global__ __launch_bounds__(kExpandBlock) void k_expand(SArgs S, DevTables T, int want_state) {
   extern __shared__ int32_t lds[];
   int32_t* sp = lds;                                          // [n][MM] job-major
-  uint8_t* pl = reinterpret_cast<uint8_t*>(lds + MM * T.n);    // [n][block] own columns
+  uint8_t* pl = reinterpret_cast<uint8_t*>(lds + MM * T.n);    // [n][64] columns
+  // the suffix wave's results for the prefix wave: jobs, work, tails
+  int32_t* sx = lds + MM * T.n + T.n * (kExpandParents / 4);   // [NW + 2 MM][64]
   const Ctrl* C = S.ctrl;
-  // the grid covers the parent capacity, so a thread has at most one
+  // the grid covers the parent capacity, so a lane has at most one
   // parent: its stack slot and first child are loaded (at a clamped index,
   // so in bounds whatever the round's count) together with the parent count
   // and before the times are staged, and the memory round trips overlap
   const int np = C->n_parents;
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int p0 = blockIdx.x * kExpandParents, p = p0 + lane;
   const int pc = p < S.PCAP ? p : S.PCAP - 1;
   const int si_any = S.p_sel[pc], off_any = S.p_off[pc];
   issue_before_branch();
@@ -671,18 +713,15 @@ __global__ __launch_bounds__(kExpandBlock) void k_expand(SArgs S, DevTables T, i
     if (threadIdx.x == 0) S.ctrl->sel_ticket = 0;
   }
   // blocks past the round's parents leave before staging
-  if (static_cast<int>(blockIdx.x * blockDim.x) >= np) return;
+  if (p0 >= np) return;
   const bool mine_p = p < np;
   const int si = mine_p ? si_any : 0;
   const int off = mine_p ? off_any : 0;
-  stage_times<MM>(T, sp);
-  __syncthreads();
   const int n = S.n, m = S.m, P = S.P;
-  const int lane = threadIdx.x & 63;
-  const size_t PH = static_cast<size_t>(S.PCAP);  // rows of the scheduled jobs, as ChildSource reads them
-  long long work = 0;
-  if (mine_p) {
-    const int l1 = S.s_l1[si], l2 = S.s_l2[si], cost = S.s_cost[si];
+  const int l1_any = S.s_l1[si], l2_any = S.s_l2[si];
+  const int l1 = mine_p ? l1_any : -1, l2 = mine_p ? l2_any : n;  // idle lanes: no steps
+  if (wave == 0) {
+    const int cost = S.s_cost[si];
     // loads of a chunk all issue before its stores (the arrays may alias as
     // far as the compiler knows)
     for (int i0 = 0; i0 < n; i0 += 32) {
@@ -693,65 +732,98 @@ __global__ __launch_bounds__(kExpandBlock) void k_expand(SArgs S, DevTables T, i
 #pragma unroll
       for (int u = 0; u < 32; ++u)
         if (i0 + u < n) {
-          S.p_perm[static_cast<size_t>(i0 + u) * S.PCAP + p] = static_cast<uint8_t>(v[u]);
-          pl[(i0 + u) * kExpandBlock + threadIdx.x] = static_cast<uint8_t>(v[u]);
+          if (mine_p) S.p_perm[static_cast<size_t>(i0 + u) * S.PCAP + p] = static_cast<uint8_t>(v[u]);
+          pl[(i0 + u) * kExpandParents + lane] = static_cast<uint8_t>(v[u]);
         }
     }
-    S.p_l1[p] = l1;
-    S.p_l2[p] = l2;
-    S.p_cost[p] = cost;
+    if (mine_p) {
+      S.p_l1[p] = l1;
+      S.p_l2[p] = l2;
+      S.p_cost[p] = cost;
+    }
+  }
+  if (T.pr != nullptr) {
+    // sixteen machines of a job per load, all in flight at once
+    constexpr int RS = MM <= 16 ? 16 : 32;
+    for (int u = threadIdx.x; u < n * (RS / 16); u += kExpandBlock) {
+      const int4 v = T.pr[u];
+      const uint32_t w[4] = {static_cast<uint32_t>(v.x), static_cast<uint32_t>(v.y),
+                             static_cast<uint32_t>(v.z), static_cast<uint32_t>(v.w)};
+      const int j = u / (RS / 16), k0 = 16 * (u % (RS / 16));
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (k0 + i < MM) sp[j * MM + k0 + i] = (w[i >> 2] >> (8 * (i & 3))) & 0xff;
+    }
+  } else {
+    stage_times<MM>(T, sp);
+  }
+  __syncthreads();
+  const size_t PH = static_cast<size_t>(S.PCAP);  // rows of the scheduled jobs, as ChildSource reads them
+  int x[MM], wk[MM];  // heads, or tails
+  uint32_t sm[NW];
+  const int d1 = l1 + 1, d2 = n - l2;
+  if (want_state) {
+    // the parent's heads and tails (no R0/Q0 substitution: that depends on
+    // the child's own prefix and suffix), scheduled jobs and their work
+#pragma unroll
+    for (int k = 0; k < MM; ++k) x[k] = wk[k] = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) sm[w] = 0;
+    const bool work = want_state == 2;
+    if (wave == 0)
+      expand_run<MM, NW>(sp, pl + lane, 0, 1, d1, work, sm, wk,
+                         [&](const int(&pk)[MM]) { head_step<MM>(x, pk); },
+                         [&](const int(&pa)[MM], const int(&pb)[MM]) { head_step2<MM>(x, pa, pb); });
+    else
+      expand_run<MM, NW>(sp, pl + lane, n - 1, -1, d2, work, sm, wk,
+                         [&](const int(&pk)[MM]) { tail_step<MM>(x, pk); },
+                         [&](const int(&pa)[MM], const int(&pb)[MM]) { tail_step2<MM>(x, pa, pb); });
+    if (mine_p) store_row<MM>(wave == 0 ? S.p_hr : S.p_hq, p, x);
+    if (wave == 1) {
+#pragma unroll
+      for (int w = 0; w < NW; ++w) sx[w * 64 + lane] = static_cast<int>(sm[w]);
+      if (work) {
+#pragma unroll
+        for (int k = 0; k < MM; ++k) sx[(NW + k) * 64 + lane] = wk[k];
+      }
+      if constexpr (FEAT) {
+#pragma unroll
+        for (int k = 0; k < MM; ++k) sx[(NW + MM + k) * 64 + lane] = x[k];
+      }
+    }
+  }
+  // child descriptors: the BEGIN side (and a simple parent's two leaves) by
+  // the first wave, the END side by the second
+  if (mine_p) {
     const int tag = p << 9, u = l2 - l1 - 1;
+    if (wave == 0) {
+      for (int c = 0; c < u; ++c) S.c_desc[off + c] = tag | (l1 + 1 + c);
+    } else if (u != 2) {
+      for (int c = 0; c < u; ++c) S.c_desc[off + u + c] = tag | (1 << 8) | (l1 + 1 + c);
+    }
+  }
+  long long work = 0;
+  if (wave == 1 && mine_p) {
     // algorithmic bound work of the children: per child with prefix d1,
     // suffix d2 and u free jobs, P(n + 4u + 4) + 2m d1 + m(m+1) d2 int ops
-    const long long d1 = l1 + 1, d2 = n - l2;
-    const long long mm1 = static_cast<long long>(m) * (m + 1);
-    if (d1 + d2 == n - 2) {  // simple parent: two leaves, BEGIN side
-      S.c_desc[off] = tag | (l1 + 1);
-      S.c_desc[off + 1] = tag | (l1 + 2);
-      work += 2 * (P * (n + 4LL) + 2LL * m * (d1 + 2) + mm1 * d2);
-    } else {                 // BEGIN children then END children
-      for (int c = 0; c < u; ++c) S.c_desc[off + c] = tag | (l1 + 1 + c);
-      for (int c = 0; c < u; ++c) S.c_desc[off + u + c] = tag | (1 << 8) | (l1 + 1 + c);
+    const long long u = l2 - l1 - 1, mm1 = static_cast<long long>(m) * (m + 1);
+    if (d1 + d2 == n - 2) {
+      work = 2 * (P * (n + 4LL) + 2LL * m * (d1 + 2) + mm1 * d2);
+    } else {
       const long long base = P * (n + 4 * (u - 1LL) + 4);
-      work += u * (base + 2LL * m * (d1 + 1) + mm1 * d2) + u * (base + 2LL * m * d1 + mm1 * (d2 + 1));
+      work = u * (base + 2LL * m * (d1 + 1) + mm1 * d2) + u * (base + 2LL * m * d1 + mm1 * (d2 + 1));
     }
-    if (want_state) {
-      // the parent's heads and tails (no R0/Q0 substitution: that depends on
-      // the child's own prefix and suffix), scheduled jobs and their work
-      int r[MM], q[MM], wk[MM];
-      uint32_t sm[NW];
+  }
+  if (want_state) {
+    __syncthreads();
+    if (wave == 0 && mine_p) {
 #pragma unroll
-      for (int k = 0; k < MM; ++k) r[k] = q[k] = wk[k] = 0;
+      for (int w = 0; w < NW; ++w) S.p_hm[w * PH + p] = sm[w] | static_cast<uint32_t>(sx[w * 64 + lane]);
+      if (want_state == 2) {
 #pragma unroll
-      for (int w = 0; w < NW; ++w) sm[w] = 0;
-      const uint8_t* mine = pl + threadIdx.x;
-      int jn = l1 >= 0 ? mine[0] : 0;
-      for (int i = 0; i <= l1; ++i) {
-        const int j = jn;
-        if (i + 1 <= l1) jn = mine[(i + 1) * kExpandBlock];
-        set_job_bit<NW>(sm, j);
-        int pk[MM];
-        job_row<MM>(sp, j, pk);
-        head_step<MM>(r, pk);
-#pragma unroll
-        for (int k = 0; k < MM; ++k) wk[k] += pk[k];
+        for (int k = 0; k < MM; ++k) wk[k] += sx[(NW + k) * 64 + lane];
+        store_row<MM>(S.p_hw, p, wk);
       }
-      jn = l2 < n ? mine[(n - 1) * kExpandBlock] : 0;
-      for (int i = n - 1; i >= l2; --i) {
-        const int j = jn;
-        if (i - 1 >= l2) jn = mine[(i - 1) * kExpandBlock];
-        set_job_bit<NW>(sm, j);
-        int pk[MM];
-        job_row<MM>(sp, j, pk);
-        tail_step<MM>(q, pk);
-#pragma unroll
-        for (int k = 0; k < MM; ++k) wk[k] += pk[k];
-      }
-      store_row<MM>(S.p_hr, p, r);
-      store_row<MM>(S.p_hq, p, q);
-      store_row<MM>(S.p_hw, p, wk);
-#pragma unroll
-      for (int w = 0; w < NW; ++w) S.p_hm[w * PH + p] = sm[w];
       // selector features of the parent (the feature kernel's definition and
       // fragment layout; used with m == MM so every index is a constant): per
       // machine head (or R0), tail (or Q0), remaining work, head + work,
@@ -760,8 +832,8 @@ __global__ __launch_bounds__(kExpandBlock) void k_expand(SArgs S, DevTables T, i
         int h[MM], tl[MM], rw[MM];
 #pragma unroll
         for (int k = 0; k < MM; ++k) {
-          h[k] = l1 >= 0 ? r[k] : ld_const(T.R0, k);
-          tl[k] = l2 < n ? q[k] : ld_const(T.Q0, k);
+          h[k] = l1 >= 0 ? x[k] : ld_const(T.R0, k);
+          tl[k] = l2 < n ? sx[(NW + MM + k) * 64 + lane] : ld_const(T.Q0, k);
           rw[k] = ld_const(T.ptot, k) - wk[k];
         }
         const int b = p >> 5, c = p & 31;
@@ -775,9 +847,9 @@ __global__ __launch_bounds__(kExpandBlock) void k_expand(SArgs S, DevTables T, i
               const int f = 8 * t + 4 * half + i, g = f / MM, k = f % MM;
               if (f < 5 * MM) {
                 const int v = g == 0 ? h[k] : g == 1 ? tl[k] : g == 2 ? rw[k] : g == 3 ? h[k] + rw[k] : rw[k] + tl[k];
-                const float x = static_cast<float>(v) * S.x_inv_scale;
-                if (S.x_f32) S.x_f32[static_cast<size_t>(f) * S.x_ld + p] = x;
-                uint32_t u = __float_as_uint(x);
+                const float xf = static_cast<float>(v) * S.x_inv_scale;
+                if (S.x_f32) S.x_f32[static_cast<size_t>(f) * S.x_ld + p] = xf;
+                uint32_t u = __float_as_uint(xf);
                 u += 0x7FFFu + ((u >> 16) & 1u);  // BF16, round to nearest even
                 w2[i >> 1] |= (u >> 16) << (16 * (i & 1));
               }
@@ -789,18 +861,21 @@ __global__ __launch_bounds__(kExpandBlock) void k_expand(SArgs S, DevTables T, i
       }
     }
   }
-  for (int d = 32; d >= 1; d >>= 1) work += __shfl_xor(work, d, 64);
-  if (lane == 0 && work)
-    atomicAdd(reinterpret_cast<unsigned long long*>(&S.ctrl->stats[kStWork]),
-              static_cast<unsigned long long>(work));
+  if (wave == 1) {
+    for (int d = 32; d >= 1; d >>= 1) work += __shfl_xor(work, d, 64);
+    if (lane == 0 && work)
+      atomicAdd(reinterpret_cast<unsigned long long*>(&S.ctrl->stats[kStWork]),
+                static_cast<unsigned long long>(work));
+  }
 }
 
 hipError_t launch_expand(const wsbb_ctx* ctx, const SArgs& A, int want_state, hipStream_t st) {
   const int m = ctx->T.m, n = ctx->T.n;
   const int mm = m <= 8 ? 8 : (m <= 12 ? 12 : (m <= 16 ? 16 : (m <= 20 ? 20 : 24)));
   const int nw = n <= 32 ? 1 : (n <= 64 ? 2 : 4);
-  const dim3 grid((A.PCAP + kExpandBlock - 1) / kExpandBlock), block(kExpandBlock);
-  const size_t shmem = sizeof(int32_t) * mm * n + static_cast<size_t>(n) * kExpandBlock;
+  const dim3 grid((A.PCAP + kExpandParents - 1) / kExpandParents), block(kExpandBlock);
+  const size_t shmem = sizeof(int32_t) * mm * n + static_cast<size_t>(n) * kExpandParents +
+                       sizeof(int32_t) * 64 * (nw + 2 * mm);
   // feature output only where the constant-index form applies (m == MM)
   const bool feat = (A.x_frag != nullptr || A.x_f32 != nullptr);
   if (feat && m != mm) return hipErrorInvalidValue;
@@ -1563,7 +1638,11 @@ static hipError_t launch_round(wsbb_ctx* ctx, const SArgs& A, int kind, hipEvent
     Ax.x_fsteps = selector_fsteps(ctx);
     Ax.x_inv_scale = 1.0f / static_cast<float>(ctx->inst.path_bound);
   }
-  hipError_t e = launch_expand(ctx, Ax, (want_state || feat_in_expand) ? 1 : 0, st);
+  // the matrix-core form sums the free jobs' work itself; the scans and the
+  // features read the scheduled jobs'
+  const bool want_work = feat_in_expand || !ctx->mfma_for() || kind == WSBB_LB1 ||
+                         selector_log_stride(ctx) > 0;
+  hipError_t e = launch_expand(ctx, Ax, want_work && (want_state || feat_in_expand) ? 2 : want_state ? 1 : 0, st);
   if (e != hipSuccess) return e;
   ChildSource src{A.p_perm, A.p_l1, A.p_l2, A.c_desc, A.PCAP, A.CCAP};
   if (want_state) {
