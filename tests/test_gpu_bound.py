@@ -218,3 +218,23 @@ def test_lb2_large_batches_in_several_launches(tid, N):
         eng.set_launch(groups=0, grid_blocks=100)
         assert np.array_equal(eng.bound(permT, l1, l2), got)
     assert np.array_equal(got[idx], ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", [oracle.LB2, oracle.LB1])
+def test_host_batches_about_the_in_place_limit(kind):
+    """Host batches that the kernel reads in place (20 jobs: up to 32768
+    nodes), just above it, and small ones after large ones on one engine."""
+    p = oracle.taillard(11)[3]
+    n = p.shape[1]
+    ref = oracle.Oracle(p)
+    with wsbb_amd.Engine(p) as eng:
+        for seed, N in enumerate((1, 32768, 65, 32769, 32767, 3)):
+            permT, l1, l2 = wsbb_amd.random_nodes(n, N, 100 + seed)
+            idx = np.unique(np.r_[0:min(N, 300), max(0, N - 300):N])
+            want = ref.bound_batch(permT[:, idx], l1[idx], l2[idx], kind=kind, threads=16)
+            assert np.array_equal(eng.bound(permT, l1, l2, kind=kind)[idx], want), (seed, N)
+            bad = permT.copy()
+            bad[n - 1, N - 1] = n
+            with pytest.raises(wsbb_amd.WsbbError, match=f"index {n * N - 1}"):
+                eng.bound(bad, l1, l2, kind=kind)

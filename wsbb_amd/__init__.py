@@ -60,8 +60,10 @@ def _load():
         "wsbb_destroy": ([_vp], ctypes.c_int),
         "wsbb_info": ([_vp, _i32p, _i32p, _i32p, _i32p], ctypes.c_int),
         "wsbb_bound_batch": ([_vp, _u8p, _i32p, _i32p, ctypes.c_int, ctypes.c_int, ctypes.c_int, _i32p], ctypes.c_int),
-        "wsbb_bound_batch_ex": ([_vp, _u8p, _i32p, _i32p, ctypes.c_int, ctypes.c_int, ctypes.c_int,
-                                 _i32p, _i32p, _i32p, _u32p, _f32p], ctypes.c_int),
+        # plain addresses: a typed pointer object per argument costs a small
+        # batch more than its kernel
+        "wsbb_bound_batch_ex": ([_vp, _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                 _vp, _vp, _vp, _vp, _vp], ctypes.c_int),
         "wsbb_bound_device": ([_vp, _vp, _vp, _vp, ctypes.c_int, ctypes.c_int, _vp], ctypes.c_int),
         "wsbb_bound_batch_noalloc": ([_vp, _u8p, _i32p, _i32p, ctypes.c_int, ctypes.c_int,
                                       ctypes.c_int, _i32p], ctypes.c_int),
@@ -135,6 +137,10 @@ lib = _load()
 
 def _p(a, t=_i32p):
     return None if a is None else a.ctypes.data_as(t)
+
+
+def _at(a):
+    return None if a is None else a.ctypes.data
 
 
 def _check(rc, what=""):
@@ -236,16 +242,15 @@ class Engine:
         l2 = np.ascontiguousarray(l2, np.int32)
         N = l1.shape[0]
         assert permT.shape == (self.n, N) and l2.shape == (N,)
-        out = np.zeros(N, np.int32)
+        out = np.empty(N, np.int32)
         am = np.zeros(N, np.int32) if argmax else None
         pv = np.zeros((self.P, N), np.int32) if pairv else None
         ft = np.zeros((5 * self.m, N), np.float32) if feat else None
         if sel is not None:
             sel = np.ascontiguousarray(sel, np.uint32)
             assert sel.shape == ((self.P + 31) // 32, N)
-        _check(lib.wsbb_bound_batch_ex(self.h, _p(permT, _u8p), _p(l1), _p(l2), N, kind, best,
-                                       _p(out), _p(am), _p(pv), _p(sel, _u32p), _p(ft, _f32p)),
-               "bound")
+        _check(lib.wsbb_bound_batch_ex(self.h, _at(permT), _at(l1), _at(l2), N, kind, best,
+                                       _at(out), _at(am), _at(pv), _at(sel), _at(ft)), "bound")
         if not (argmax or pairv or feat):
             return out
         res = {"bound": out}

@@ -336,6 +336,7 @@ int wsbb_destroy(wsbb_ctx* ctx) {
   destroy_selector(ctx);
   ctx->tables.release();
   ctx->batch.release();
+  ctx->pinned.release();
   if (ctx->ev_start) (void)hipEventDestroy(ctx->ev_start);
   if (ctx->ev_stop) (void)hipEventDestroy(ctx->ev_stop);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -352,16 +353,33 @@ int wsbb_info(const wsbb_ctx* ctx, int* n, int* m, int* pairs, int* num_cus) {
   return WSBB_OK;
 }
 
+// Plain host batches up to this size are copied by the host into pinned memory
+// that the kernel reads and writes in place: every node is read once, so the
+// transfer is the kernel's own loads, and a call is one launch and one wait.
+// Above it copies into device memory win (their transfer runs ahead of the
+// kernel instead of inside it).  In place / copied, whole calls in us: 20x5 64
+// nodes 23.7 / 39.8, 20x10 4096 31.8 / 49.4, 30000 (0.96 MB) 88 / 99, 60000
+// 163 / 159, 50x20 14000 (0.87 MB) 108 / 113, 60000 360 / 272.  (Copied, and
+// with the argument checks below leaving at the first fault: 49.9 and 74.6.)
+constexpr size_t kPinnedBytes = size_t(1) << 20;
+
+// Whole passes without an exit (which the compiler vectorises); the first
+// offender is looked for only when there is one.
 static int check_nodes_host(const wsbb_ctx* ctx, const uint8_t* permT,
                             const int32_t* l1, const int32_t* l2, int N) {
   const int n = ctx->T.n;
-  for (int k = 0; k < N; ++k) {
+  int bad = 0;
+  for (int k = 0; k < N; ++k) bad |= (l1[k] < -1) | (l2[k] > n) | (l2[k] <= l1[k]);
+  for (int k = 0; bad && k < N; ++k) {
     if (l1[k] < -1 || l2[k] > n || l2[k] <= l1[k]) {
       set_error("node " + std::to_string(k) + ": limits out of range");
       return WSBB_EINVAL;
     }
   }
-  for (size_t i = 0; i < static_cast<size_t>(n) * N; ++i)
+  const size_t bytes = static_cast<size_t>(n) * N;
+  uint8_t top = 0;
+  for (size_t i = 0; i < bytes; ++i) top = permT[i] > top ? permT[i] : top;
+  for (size_t i = 0; top >= n && i < bytes; ++i)
     if (permT[i] >= n) {
       set_error("job id out of range at position-major index " + std::to_string(i));
       return WSBB_EINVAL;
@@ -392,15 +410,26 @@ int wsbb_bound_batch_ex(wsbb_ctx* ctx, const uint8_t* permT, const int32_t* l1,
   const size_t o_feat = o_sel + (sel ? al(size_t(4) * nsw * N) : 0);
   const size_t total = o_feat + (feat ? al(size_t(4) * 5 * m * N) : 0);
   WSBB_HIP(hipSetDevice(ctx->device), "hipSetDevice");
-  WSBB_HIP(ctx->batch.reserve(total), "hipMalloc(batch)");
   hipStream_t st = ctx->stream;
-  WSBB_HIP(hipMemcpyAsync(ctx->batch.as<char>(o_perm), permT, size_t(n) * N, hipMemcpyHostToDevice, st), "H2D perm");
-  WSBB_HIP(hipMemcpyAsync(ctx->batch.as<char>(o_l1), l1, size_t(4) * N, hipMemcpyHostToDevice, st), "H2D l1");
-  WSBB_HIP(hipMemcpyAsync(ctx->batch.as<char>(o_l2), l2, size_t(4) * N, hipMemcpyHostToDevice, st), "H2D l2");
+  const bool pinned = !argmax && !pairv && !sel && !feat && total <= kPinnedBytes &&
+                      ctx->pinned.reserve(kPinnedBytes);  // whole: an allocation costs 40 us at any size
+  char* base;  // of the nodes and results, as the kernel sees them
+  if (pinned) {
+    base = ctx->pinned.dev;
+    memcpy(ctx->pinned.ptr + o_perm, permT, size_t(n) * N);
+    memcpy(ctx->pinned.ptr + o_l1, l1, size_t(4) * N);
+    memcpy(ctx->pinned.ptr + o_l2, l2, size_t(4) * N);
+  } else {
+    WSBB_HIP(ctx->batch.reserve(total), "hipMalloc(batch)");
+    base = ctx->batch.as<char>();
+    WSBB_HIP(hipMemcpyAsync(base + o_perm, permT, size_t(n) * N, hipMemcpyHostToDevice, st), "H2D perm");
+    WSBB_HIP(hipMemcpyAsync(base + o_l1, l1, size_t(4) * N, hipMemcpyHostToDevice, st), "H2D l1");
+    WSBB_HIP(hipMemcpyAsync(base + o_l2, l2, size_t(4) * N, hipMemcpyHostToDevice, st), "H2D l2");
+  }
   if (sel)
-    WSBB_HIP(hipMemcpyAsync(ctx->batch.as<char>(o_sel), sel, size_t(4) * nsw * N, hipMemcpyHostToDevice, st), "H2D sel");
-  BatchSource src{ctx->batch.as<uint8_t>(o_perm), ctx->batch.as<int32_t>(o_l1),
-                  ctx->batch.as<int32_t>(o_l2), N};
+    WSBB_HIP(hipMemcpyAsync(base + o_sel, sel, size_t(4) * nsw * N, hipMemcpyHostToDevice, st), "H2D sel");
+  BatchSource src{reinterpret_cast<uint8_t*>(base + o_perm), reinterpret_cast<int32_t*>(base + o_l1),
+                  reinterpret_cast<int32_t*>(base + o_l2), N};
   BoundArgs A{};
   A.N = N;
   A.kind = kind;
@@ -408,13 +437,18 @@ int wsbb_bound_batch_ex(wsbb_ctx* ctx, const uint8_t* permT, const int32_t* l1,
   A.groups = ctx->groups_for(N);
   A.pk = ctx->int16_for(N);
   ctx->johnson_args(A);
-  A.out = ctx->batch.as<int32_t>(o_out);
-  A.argmax = argmax ? ctx->batch.as<int32_t>(o_am) : nullptr;
-  A.pairv = pairv ? ctx->batch.as<int32_t>(o_pv) : nullptr;
-  A.sel = sel ? ctx->batch.as<const uint32_t>(o_sel) : nullptr;
-  A.feat = feat ? ctx->batch.as<float>(o_feat) : nullptr;
+  A.out = reinterpret_cast<int32_t*>(base + o_out);
+  A.argmax = argmax ? reinterpret_cast<int32_t*>(base + o_am) : nullptr;
+  A.pairv = pairv ? reinterpret_cast<int32_t*>(base + o_pv) : nullptr;
+  A.sel = sel ? reinterpret_cast<const uint32_t*>(base + o_sel) : nullptr;
+  A.feat = feat ? reinterpret_cast<float*>(base + o_feat) : nullptr;
   A.feat_scale = static_cast<float>(ctx->inst.path_bound > 0 ? ctx->inst.path_bound : 1);
   WSBB_HIP(launch_bound(ctx->T, src, A, ctx->grid_cap(), st), "bound kernel launch");
+  if (pinned) {
+    WSBB_HIP(hipStreamSynchronize(st), "hipStreamSynchronize");
+    memcpy(out, ctx->pinned.ptr + o_out, size_t(4) * N);
+    return WSBB_OK;
+  }
   WSBB_HIP(hipMemcpyAsync(out, A.out, size_t(4) * N, hipMemcpyDeviceToHost, st), "D2H out");
   if (argmax) WSBB_HIP(hipMemcpyAsync(argmax, A.argmax, size_t(4) * N, hipMemcpyDeviceToHost, st), "D2H argmax");
   if (pairv) WSBB_HIP(hipMemcpyAsync(pairv, A.pairv, size_t(4) * P * N, hipMemcpyDeviceToHost, st), "D2H pairv");

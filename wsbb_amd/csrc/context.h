@@ -41,6 +41,37 @@ struct DevBuf {
   }
 };
 
+// Grow-only pinned host memory that kernels read and write in place.
+struct HostBuf {
+  char* ptr = nullptr;  // as the host sees it
+  char* dev = nullptr;  // as kernels do
+  size_t bytes = 0;
+  // false: no pinned memory to be had (the caller stages by copies)
+  bool reserve(size_t need) {
+    if (need <= bytes) return true;
+    release();
+    void *h = nullptr, *d = nullptr;
+    if (hipHostMalloc(&h, need, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    if (hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
+      (void)hipGetLastError();
+      (void)hipHostFree(h);
+      return false;
+    }
+    ptr = static_cast<char*>(h);
+    dev = static_cast<char*>(d);
+    bytes = need;
+    return true;
+  }
+  void release() {
+    if (ptr) (void)hipHostFree(ptr);
+    ptr = dev = nullptr;
+    bytes = 0;
+  }
+};
+
 struct SearchState;    // search.hip
 struct SelectorState;  // selector.hip
 
@@ -62,6 +93,7 @@ struct wsbb_ctx {
   wsbb::DevTables T{};
   wsbb::DevBuf tables;  // every instance table in one allocation
   wsbb::DevBuf batch;   // staging for host-buffer batch calls
+  wsbb::HostBuf pinned; // and for the small ones
   wsbb::Launch launch;
   int pool_capacity = 1 << 24;  // device node-pool capacity (nodes)
   int profile_every = 0;         // time every k-th round's bound launch in wsbb_solve
