@@ -221,3 +221,16 @@ def test_resume_rejects_nodes_the_device_never_makes():
         # a root carrying a huge bound is still taken without an incumbent
         res = eng.resume(dict(base, cost=np.array([2**30], np.int32)), pool_size=4096)
     assert res["proven"] and res["best"] == 1278
+
+
+@pytest.mark.parametrize("n,m,high", [(31, 4, 5), (32, 9, 99), (33, 4, 5), (64, 9, 99), (65, 4, 5), (126, 5, 99)])
+def test_parents_at_the_edges_of_lane_groups(n, m, high):
+    """Pop order where a parent's positions fill 32 or 64 lanes or just pass
+    them, with many tied bounds (small times) and few."""
+    p = np.random.default_rng(n).integers(1, high + 1, size=(m, n)).astype(np.int32)
+    _, st, _, tr = oracle.Oracle(p).solve_batched(pool_size=3000, max_batches=2, budget=1500, trace=10_000)
+    _, rounds = traced_solve(p, 3000, 2, budget=1500)
+    tk = {k: v[:st["decomposed"]] for k, v in taken(tr).items()}
+    assert np.array_equal(np.concatenate([r["permT"].T for r in rounds]), tk["perm"].astype(np.uint8))
+    for key in ("l1", "l2", "cost"):
+        assert np.array_equal(np.concatenate([r[key] for r in rounds]), tk[key])

@@ -1121,35 +1121,54 @@ __device__ void settle_round(const SArgs& S, int np, int t, int* s_w16, int* s_l
   }
 }
 
-// ---- rank: one wave per parent -------------------------------------------
-// one DPP step of the leaf minimum: cost ascending, then job descending
-template <int CTRL, int RMASK>
-__device__ __forceinline__ void leaf_step(int& lmin, int& lwin, int& lwjob) {
-  const int om = __builtin_amdgcn_update_dpp(INT_MAX, lmin, CTRL, RMASK, 0xf, false);
-  const int oj = __builtin_amdgcn_update_dpp(-1, lwjob, CTRL, RMASK, 0xf, false);
-  const int ow = __builtin_amdgcn_update_dpp(-1, lwin, CTRL, RMASK, 0xf, false);
-  if (om < lmin || (om == lmin && oj > lwjob)) {
-    lmin = om;
-    lwin = ow;
-    lwjob = oj;
-  }
+// ---- rank: a group of lanes per parent -----------------------------------
+// orders a wave's own LDS writes before its later reads (LDS runs a wave's
+// accesses in order: no instruction, the compiler must not reorder them)
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+// sum over groups of 32 lanes or over the wave, in every lane
+template <int G>
+__device__ __forceinline__ int group_sum(int v) {
+  if constexpr (G == 64) return wave_reduce(v, 0, OpAdd());
+  v += WSBB_DPP(v, 0, 0x111, 0xf);
+  v += WSBB_DPP(v, 0, 0x112, 0xf);
+  v += WSBB_DPP(v, 0, 0x114, 0xf);
+  v += WSBB_DPP(v, 0, 0x118, 0xf);
+  v += WSBB_DPP(v, 0, 0x142, 0xa);
+  const int lo = __builtin_amdgcn_readlane(v, 31), hi = __builtin_amdgcn_readlane(v, 63);
+  return (threadIdx.x & 32) ? hi : lo;
 }
 
-// Four parents per block and pass.  A parent's children and the jobs at its
-// free positions are read in one round of loads (its child count is 2u, or 2
-// at depth n - 2, as expand numbered them).  The chosen side's ranks go to
-// the parent's ranked rows (child index and bound by rank), which settle and
-// push read without the child descriptors.
-constexpr int kRankWaves = 4;
+// A group's lanes hold the parent's free positions: lane i the i-th child of
+// either side (both place the job at l1 + 1 + i) and that job; 32 lanes up to
+// 32 jobs, else 64 lanes with two positions each.  The side is chosen by two
+// sums over the group; the chosen side's children are ordered by (bound, job)
+// as one word each (bounds stay below 2^19), every lane counting the smaller
+// words of its group.  The ranks go to the parent's ranked rows (child index
+// and bound by rank), which settle and push read without the child
+// descriptors.  Bound by latency: two rounds of loads, then LDS reads of four
+// words; waves wait for nothing but themselves.  (A wave per parent, a word
+// for bounds and one for jobs, four sums and a block barrier a parent: 20x20,
+// 34K parents 16.5 us, 20x10, 2900 4.7; in groups 6.8 and 4.0.)
+constexpr int kRankThreads = 256;
+inline int rank_parents(int n) { return kRankThreads / (n <= 32 ? 32 : 64); }  // of a block
 
-__global__ __launch_bounds__(256) void k_rank(SArgs S) {
-  __shared__ int s_b[kRankWaves][2 * kMaxJobs];  // children's bounds, BEGIN then END
-  __shared__ int s_job[kRankWaves][kMaxJobs];    // job at free position l1 + 1 + i
+template <int G>
+__global__ __launch_bounds__(kRankThreads) void k_rank(SArgs S) {
+  constexpr int T = G == 32 ? 1 : 2, PB = kRankThreads / G;
+  static_assert(G * T >= kMaxJobs || G == 32, "a slot per free position");
+  __shared__ __align__(16) int s_key[PB][G * T];
   Ctrl* C = S.ctrl;
-  const int np = C->n_parents;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int grp = threadIdx.x / G, gl = threadIdx.x & (G - 1);
   const int n = S.n;
+  // the first parent's fields (at a clamped index) go out with the control loads
+  int p = blockIdx.x * PB + grp;
+  int off = S.p_off[min(p, S.PCAP - 1)], l1 = S.p_l1[min(p, S.PCAP - 1)], l2 = S.p_l2[min(p, S.PCAP - 1)];
+  const int np = C->n_parents;
   const int inc0 = C->inc;
+  issue_before_branch();
   // leaf children of the block's parents: one plain store per block (the
   // settle kernel sums the blocks' counts); an atomic per wave into one
   // counter serialises when a round is all leaf parents (ten thousand waves)
@@ -1160,97 +1179,92 @@ __global__ __launch_bounds__(256) void k_rank(SArgs S) {
     if (threadIdx.x < kSettleChain * kLink) S.set_link[threadIdx.x] = 0;
     if (threadIdx.x == 0) C->set_ticket = 0;
   }
-  for (int pb = blockIdx.x * kRankWaves; pb < np; pb += gridDim.x * kRankWaves) {
-    const int p = pb + wave;
+  __syncthreads();
+  for (int pb = blockIdx.x * PB; pb < np; pb += gridDim.x * PB) {
     const bool live = p < np;
-    int off = 0, l1 = 0, u = 0, simple = 0;
-    if (live) {
+    const int u = live ? l2 - l1 - 1 : 0;
+    const bool simple = ((l1 + 1) + (n - l2)) == n - 2;
+    int b0[T], b1[T], job[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int i = gl + G * t;
+      b0[t] = b1[t] = job[t] = 0;
+      if (i < u) {
+        b0[t] = S.c_bound[off + i];
+        if (!simple) b1[t] = S.c_bound[off + u + i];
+        job[t] = S.p_perm[static_cast<size_t>(l1 + 1 + i) * S.PCAP + p];
+      }
+    }
+    // bounds of kSideBest and more are counted, the others summed: the side
+    // with more of them, then the larger sum (a simple parent has one side)
+    int d = 0, e = 0;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const bool big0 = b0[t] >= kSideBest, big1 = b1[t] >= kSideBest;
+      d += big0 - big1;
+      e += (big0 ? 0 : b0[t]) - (big1 ? 0 : b1[t]);
+    }
+    d = group_sum<G>(d);
+    e = group_sum<G>(e);
+    const int side = (d > 0 || (d == 0 && e > 0)) ? 0 : 1;
+    const int nch = simple ? (side == 0 ? u : 0) : u;
+    int key[T];
+    int below = 0;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int i = gl + G * t, c = side == 0 ? b0[t] : b1[t];
+      key[t] = i < nch ? (c << 7) | job[t] : INT_MAX;
+      s_key[grp][i] = key[t];
+      unsigned long long m = __ballot(i < nch && c < inc0);
+      if constexpr (G == 32) m = (threadIdx.x & 32) ? m >> 32 : m & 0xffffffffull;
+      below += __popcll(m);
+    }
+    wave_lds_order();
+    int rk[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) rk[t] = 0;
+    const int4* q = reinterpret_cast<const int4*>(s_key[grp]);
+    for (int k = 0; 4 * k < nch; ++k) {
+      const int4 v = q[k];
+#pragma unroll
+      for (int t = 0; t < T; ++t) rk[t] += (v.x < key[t]) + (v.y < key[t]) + (v.z < key[t]) + (v.w < key[t]);
+    }
+    int* ro = S.r_order + static_cast<size_t>(p) * n;
+    int* rc = S.r_cost + static_cast<size_t>(p) * n;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int i = gl + G * t;
+      if (i < nch) {
+        ro[rk[t]] = i;
+        rc[rk[t]] = key[t] >> 7;
+      }
+    }
+    if (live && gl == 0) {
+      int lmin = INT_MAX, lmax = INT_MAX, lwin = -1;
+      if (simple && nch > 0) {
+        // two leaves, inserted worst first (cost desc, job desc), and only a
+        // strictly better one replaces the incumbent: of equal costs the one
+        // with the larger job wins
+        const int k0 = s_key[grp][0], k1 = s_key[grp][1], c0 = k0 >> 7, c1 = k1 >> 7;
+        lmin = min(c0, c1);
+        lmax = max(c0, c1);
+        lwin = off + ((c1 < c0 || (c1 == c0 && k1 >= k0)) ? 1 : 0);
+        atomicAdd(&s_leaves, nch);
+      }
+      S.p_kept0[p] = below;
+      S.p_side[p] = side;
+      S.p_nch[p] = nch;
+      S.p_leafmin[p] = lmin;
+      S.p_leafmax[p] = lmax;
+      S.p_leafwin[p] = lwin;
+    }
+    wave_lds_order();
+    p += gridDim.x * PB;
+    if (p < np) {
       off = S.p_off[p];
       l1 = S.p_l1[p];
-      const int l2 = S.p_l2[p];
-      u = l2 - l1 - 1;
-      simple = ((l1 + 1) + (n - l2)) == n - 2;
-      const int cnt = simple ? 2 : 2 * u;
-      for (int c = lane; c < cnt; c += 64) s_b[wave][c] = S.c_bound[off + c];
-      for (int i = lane; i < u; i += 64)
-        s_job[wave][i] = S.p_perm[static_cast<size_t>(l1 + 1 + i) * S.PCAP + p];
+      l2 = S.p_l2[p];
     }
-    __syncthreads();
-    if (live) {
-      const int cnt = simple ? 2 : 2 * u;
-      int c0 = 0, c1 = 0, s0 = 0, s1 = 0;
-      for (int c = lane; c < cnt; c += 64) {
-        const int b = s_b[wave][c];
-        const int sd = simple ? 0 : (c >= u);
-        const int big = b >= kSideBest;
-        if (sd == 0) {
-          c0 += big;
-          s0 += big ? 0 : b;
-        } else {
-          c1 += big;
-          s1 += big ? 0 : b;
-        }
-      }
-      c0 = wave_reduce(c0, 0, OpAdd());
-      c1 = wave_reduce(c1, 0, OpAdd());
-      s0 = wave_reduce(s0, 0, OpAdd());
-      s1 = wave_reduce(s1, 0, OpAdd());
-      const int side = (c0 > c1) ? 0 : (c1 > c0) ? 1 : (s0 > s1) ? 0 : 1;
-      const int nch = simple ? (side == 0 ? 2 : 0) : u;
-      // the i-th child of either side (and of a simple parent) places the
-      // job at position l1 + 1 + i
-      const int* sb = &s_b[wave][simple ? 0 : side * u];
-      int* ro = S.r_order + static_cast<size_t>(p) * n;
-      int* rc = S.r_cost + static_cast<size_t>(p) * n;
-      int lmin = INT_MAX, lwin = -1, lwjob = -1, lmax = INT_MIN, below = 0;
-      for (int i = lane; i < nch; i += 64) {
-        const int cc = sb[i], jj = s_job[wave][i];
-        int rk = 0;
-        for (int k = 0; k < nch; ++k) {
-          const int ck = sb[k];
-          rk += (ck < cc) || (ck == cc && s_job[wave][k] < jj);
-        }
-        ro[rk] = i;
-        rc[rk] = cc;
-        below += cc < inc0;
-        if (simple) {
-          // leaves are inserted worst first (cost desc, job desc) and only a
-          // strictly better one replaces the incumbent: among equal minima
-          // the one with the larger job id wins
-          if (cc < lmin || (cc == lmin && jj > lwjob)) {
-            lmin = cc;
-            lwin = off + i;
-            lwjob = jj;
-          }
-          lmax = max(lmax, cc);
-        }
-      }
-      if (simple) {
-        // scan of (cost ascending, job descending) with the child index as
-        // payload, same DPP steps as wave_incl_scan
-        leaf_step<0x111, 0xf>(lmin, lwin, lwjob);
-        leaf_step<0x112, 0xf>(lmin, lwin, lwjob);
-        leaf_step<0x114, 0xf>(lmin, lwin, lwjob);
-        leaf_step<0x118, 0xf>(lmin, lwin, lwjob);
-        leaf_step<0x142, 0xa>(lmin, lwin, lwjob);
-        leaf_step<0x143, 0xc>(lmin, lwin, lwjob);
-        lmin = __builtin_amdgcn_readlane(lmin, 63);
-        lwin = __builtin_amdgcn_readlane(lwin, 63);
-        lwjob = __builtin_amdgcn_readlane(lwjob, 63);
-        lmax = wave_reduce(lmax, INT_MIN, OpMax());
-      }
-      below = wave_reduce(below, 0, OpAdd());
-      if (lane == 0) {
-        S.p_kept0[p] = below;
-        S.p_side[p] = side;
-        S.p_nch[p] = nch;
-        S.p_leafmin[p] = simple ? lmin : INT_MAX;
-        S.p_leafmax[p] = (simple && nch > 0) ? lmax : INT_MAX;
-        S.p_leafwin[p] = simple ? lwin : -1;
-        if (simple && nch > 0) atomicAdd(&s_leaves, nch);
-      }
-    }
-    __syncthreads();
   }
   __syncthreads();
   if (threadIdx.x == 0) S.r_leaves[blockIdx.x] = s_leaves;
@@ -1285,25 +1299,31 @@ __global__ __launch_bounds__(1024) void k_settle_chain(SArgs S) {
   settle_round<true>(S, np, t, s_w16, &s_last, s_pre);
 }
 
-// ---- push survivors: one wave per parent ------------------------------------
+// ---- push survivors: a group of lanes per parent ----------------------------
 // A parent's kept children are its first `kept` ranks; the rank-k child goes
 // to stack slot base + total - 1 - (koff + k), so the round's first parent's
 // best child ends on top.  A parent's fields, its permutation column and its
 // ranked rows are read in one round of loads (rows are read whole, n entries,
-// whatever the kept count); lane k then writes the rank-k child.
-__global__ __launch_bounds__(256) void k_push(SArgs S) {
-  __shared__ int s_col[4][kMaxJobs];
+// whatever the kept count); lane k then writes the rank-k child.  Groups as in
+// the rank kernel: neighbouring parents' survivors are neighbours in the
+// stack, so a wave's store of one position covers two parents' bytes (a wave
+// per parent, bytes one by one from LDS: 20x20, 34K parents 12 us, now 8.2).
+template <int G>
+__global__ __launch_bounds__(kRankThreads) void k_push(SArgs S) {
+  constexpr int T = G == 32 ? 1 : 2, PB = kRankThreads / G;
+  __shared__ __align__(16) uint8_t s_col[PB][G * T];
   const Ctrl* C = S.ctrl;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int grp = threadIdx.x / G, gl = threadIdx.x & (G - 1);
   const int n = S.n;
-  const int stride = gridDim.x * 4;
+  const int stride = gridDim.x * PB;
   // a parent's loads depend only on its index: the first pass's (at an
   // index clamped to the capacity) go out with the control loads
   bool first = true;
   int kept = 0, koff = 0, side = 0, pl1 = 0, pl2 = 0;
-  // positions / ranks lane and lane + 64 (n <= 128)
-  int ord[2] = {0, 0}, cst[2] = {0, 0};
-  uint32_t col[2] = {0u, 0u};  // a register per byte: no wait before the control loads
+  int ord[T], cst[T];
+  uint32_t col[T];  // a register per byte: no wait before the control loads
+#pragma unroll
+  for (int t = 0; t < T; ++t) ord[t] = cst[t] = 0, col[t] = 0u;
   auto load = [&](int p) {
     kept = S.p_kept[p];
     koff = S.p_koff[p];
@@ -1313,8 +1333,8 @@ __global__ __launch_bounds__(256) void k_push(SArgs S) {
     const int* ro = S.r_order + static_cast<size_t>(p) * n;
     const int* rc = S.r_cost + static_cast<size_t>(p) * n;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int k = lane + 64 * t;
+    for (int t = 0; t < T; ++t) {
+      const int k = gl + G * t;
       if (k < n) {
         col[t] = S.p_perm[static_cast<size_t>(k) * S.PCAP + p];
         ord[t] = ro[k];
@@ -1325,34 +1345,40 @@ __global__ __launch_bounds__(256) void k_push(SArgs S) {
   // after an overflow or at the end of the search select left no parents
   const int np = C->n_parents, base = C->push_base, total = C->push_total;
   {
-    const int p0 = blockIdx.x * 4 + wave;
+    const int p0 = blockIdx.x * PB + grp;
     load(p0 < S.PCAP ? p0 : S.PCAP - 1);
   }
   issue_before_branch();
-  for (int pb = blockIdx.x * 4; pb < np; pb += stride) {
-    const int p = pb + wave;
+  for (int pb = blockIdx.x * PB; pb < np; pb += stride) {
+    const int p = pb + grp;
     const bool live = p < np;
     if (!first && live) load(p);
     first = false;
-    if (live) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
-        if (lane + 64 * t < n) s_col[wave][lane + 64 * t] = static_cast<int>(col[t]);
-    }
-    __syncthreads();
+    for (int t = 0; t < T; ++t) s_col[grp][gl + G * t] = static_cast<uint8_t>(col[t]);
+    wave_lds_order();
     if (live) {
       const int sw0 = side == 0 ? pl1 + 1 : pl2 - 1;
       int l1 = pl1 + (side == 0), l2 = pl2 - (side == 1);
       if (l2 - l1 == 2) l1 += 1;  // the last free job is placed too (limites_set)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int k = lane + 64 * t;
+      for (int t = 0; t < T; ++t) {
+        const int k = gl + G * t;
         if (k < kept) {
           const int j = pl1 + 1 + ord[t];
           const int slot = base + total - 1 - (koff + k);
-          for (int i = 0; i < n; ++i) {
-            const int src = (i == sw0) ? j : ((i == j) ? sw0 : i);
-            S.s_perm[static_cast<size_t>(i) * S.CAP + slot] = static_cast<uint8_t>(s_col[wave][src]);
+          const int cj = s_col[grp][j], cs = s_col[grp][sw0];  // change places
+          uint8_t* to = S.s_perm + slot;
+          for (int i0 = 0; i0 < n; i0 += 16) {
+            const int4 q = *reinterpret_cast<const int4*>(&s_col[grp][i0]);
+            const int w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              if (i0 + i >= n) break;
+              const int c = w[i >> 2] >> (8 * (i & 3));
+              *to = static_cast<uint8_t>(i0 + i == sw0 ? cj : i0 + i == j ? cs : c);
+              to += S.CAP;
+            }
           }
           S.s_l1[slot] = l1;
           S.s_l2[slot] = l2;
@@ -1361,7 +1387,7 @@ __global__ __launch_bounds__(256) void k_push(SArgs S) {
         }
       }
     }
-    __syncthreads();
+    wave_lds_order();
   }
 }
 
@@ -1611,8 +1637,7 @@ static int ensure_search(wsbb_ctx* ctx, int pool_size, int max_batches, int cap_
 static hipError_t launch_round(wsbb_ctx* ctx, const SArgs& A, int kind, hipEvent_t ev0,
                                hipEvent_t ev1) {
   hipStream_t st = ctx->stream;
-  const int rblocks = (A.PCAP + kRankWaves - 1) / kRankWaves;
-  const int pblocks = (A.PCAP + 3) / 4;
+  const int gblocks = (A.PCAP + rank_parents(A.n) - 1) / rank_parents(A.n);  // rank, push
   // large pools: the chained select over several CUs
   if (static_cast<long long>(A.pool_m1) * A.max_batches > 16LL * kSelWin0)
     hipLaunchKernelGGL(k_select_chain, dim3(kSelChain), dim3(1024), 0, st, A);
@@ -1755,13 +1780,16 @@ static hipError_t launch_round(wsbb_ctx* ctx, const SArgs& A, int kind, hipEvent
       hipLaunchKernelGGL(k_log_advance, dim3(1), dim3(1), 0, st, L);
     }
   }
-  hipLaunchKernelGGL(k_rank, dim3(rblocks < kRankGrid ? rblocks : kRankGrid), dim3(256), 0, st, A);
+  const dim3 ggrid(gblocks < kRankGrid ? gblocks : kRankGrid), gblock(kRankThreads);
+  if (A.n <= 32) hipLaunchKernelGGL(k_rank<32>, ggrid, gblock, 0, st, A);
+  else hipLaunchKernelGGL(k_rank<64>, ggrid, gblock, 0, st, A);
   // more parents than one settle chunk: the chunks on kSettleChain blocks
   if (A.PCAP > kSettleChunk && A.PCAP <= kSettleChain * kChainChunk)
     hipLaunchKernelGGL(k_settle_chain, dim3(kSettleChain), dim3(1024), 0, st, A);
   else
     hipLaunchKernelGGL(k_settle, dim3(1), dim3(1024), 0, st, A);
-  hipLaunchKernelGGL(k_push, dim3(pblocks < 4096 ? pblocks : 4096), dim3(256), 0, st, A);
+  if (A.n <= 32) hipLaunchKernelGGL(k_push<32>, ggrid, gblock, 0, st, A);
+  else hipLaunchKernelGGL(k_push<64>, ggrid, gblock, 0, st, A);
   return hipGetLastError();
 }
 
