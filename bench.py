@@ -4,11 +4,12 @@
 Headline (one step = one bound launch): Taillard ta051, 50 jobs x 20
 machines, int32 times in [1, 99]; a batch of 2^20 synthetic nodes (prefix
 and suffix lengths uniform so the scheduled depth is in [0, 49], random job
-permutations) resident in HBM, bounded with plain LB2 by the int32 kernel
-with autotuned launch shape.  `value` is nodes bounded per second over the K
+permutations) resident in HBM, bounded with plain LB2 in int32 values (the
+sums of the Johnson scan as exact int8 matrix products) with autotuned launch
+shape.  `value` is nodes bounded per second over the K
 timed launches; `roofline` relates the algorithmic integer work of the batch
 to the kernel's launch time (HIP events on the context stream) and the int32
-VALU peak.
+VALU peak; the matrix cores carry most of that work, so it can exceed one.
 
 Sub-objects: "int16_two_node" (the same batch by the two-node int16 kernel,
 against the packed 16-bit issue rate), "config1" (ta001-ta010, 20x5, solved
@@ -658,12 +659,13 @@ def main():
                           "nodes_per_s": bt["N"] / (bt["ms"] / 1e3)}), flush=True)
         return
 
-    rf = roofline(bt, PEAK_VALU_TOPS, "bound_kernel<20, 2, 0, 256, BatchSource> (int32)")
+    rf = roofline(bt, PEAK_VALU_TOPS, "k_johnson<20, 2, 13, ...> (int8 matrix products, int32 sums "
+                  "and values; the scan's operations over the VALU peak, which it can exceed)")
     rf["traffic"] = measured_traffic("batched_int32")
     # the derived peak against the probe kernel's measured rates on this GPU
     rf["peak_check"] = {"measured_tlaneops": valu_peak(wsbb_amd),
                         "derived": "256 CU x 64 lanes x 2.4 GHz = 39.3 T int32 lane-ops/s",
-                        "scan_instructions": "v_bfe_u32, v_mad_i32_i24, v_mad_u32_u24, v_max_i32"}
+                        "scan_instructions": "v_mfma_i32_32x32x32_i8, v_max3_i32"}
     line = {
         "metric": "LB2 bounded nodes/s + time-to-proven-optimum, 1 MI355X vs host CPU",
         "value": bt["N"] / (bt["wall_ms"] / 1e3),

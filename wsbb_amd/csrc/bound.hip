@@ -1,4 +1,7 @@
-// Node bound kernels for the permutation flowshop on gfx950.
+// Node bound kernels for the permutation flowshop on gfx950.  Plain LB2, whole
+// or over tile subsets, runs on the matrix cores (johnson.hip) wherever times
+// fit a signed byte and n <= 126; the scans here take other instances, LB1,
+// features, argmax, pair values and masks, and the int16 form.
 //
 // One lane bounds one node.  All lanes of a wavefront walk the same machine
 // pair and the same Johnson step at the same time, so every per-step constant
