@@ -57,7 +57,11 @@ constexpr int kSettleChunk = 1024 * kSettleK;  // parents per chunk of the one-b
 constexpr int kChainK = 8;     // consecutive parents per thread of the chained settle
 constexpr int kChainChunk = 1024 * kChainK;    // parents per block of the chained settle
 static_assert(kRankGrid == 4 * 1024, "each of the settle block's threads sums four rank blocks' counts");
-constexpr int kSelChain = 8;   // blocks of the chained select (large pools)
+// blocks of the chained select (large pools) and the candidates of each: a
+// window's own scan against one more hand-off; 20x20, 34K parents, 8 blocks of
+// 16384 23.8 us, 16 of 8192 20.0, 32 of 4096 28.2
+constexpr int kSelChain = 16;
+constexpr int kChainWin = 8192;
 constexpr int kLink = 8;       // ints per hand-off record: two to a word (link_put)
 constexpr int kSettleChain = 16;  // blocks of the chained settle (large pools)
 // largest cost a select key holds: bounds stay below 2^19, and a larger
@@ -540,7 +544,7 @@ __global__ __launch_bounds__(1024) void k_select(SArgs S) {
 }
 
 // ---- select for large pools: windows on kSelChain blocks ------------------
-// Block t (in the order blocks take tickets) turns window t (kSelWin
+// Block t (in the order blocks take tickets) turns window t (kChainWin
 // candidates) into words and prefix sums at once, then waits for block
 // t - 1's hand-off record (carried reservation, sub-batches, parents,
 // children, pruned, consumed, or a stop), settles its window from it and
@@ -551,8 +555,8 @@ __global__ __launch_bounds__(1024) void k_select(SArgs S) {
 // continues alone if the round needs more windows; the block where the
 // round ends commits it (select_commit).
 __global__ __launch_bounds__(1024) void k_select_chain(SArgs S) {
-  constexpr int KPER = kSelWin / 1024;
-  __shared__ int s_p[kSelWin + kSelWin / 16];
+  constexpr int KPER = kChainWin / 1024;
+  __shared__ int s_p[kSelWin + kSelWin / 16];  // the last block goes on in windows of kSelWin
   __shared__ int s_w16[80];
   __shared__ int s_state[4];
   __shared__ int s_ticket;
@@ -584,12 +588,12 @@ __global__ __launch_bounds__(1024) void k_select_chain(SArgs S) {
     }
     return;
   }
-  const int w0 = t * kSelWin;
+  const int w0 = t * kChainWin;
   if (w0 >= top) {  // no candidates in this block's window
     if (tid == 0) hand_stop();
     return;
   }
-  const int win = min(kSelWin, top - w0);
+  const int win = min(kChainWin, top - w0);
   int word[KPER];
   window_words<KPER>(S, top, inc, w0, win, s_p, s_w16, word);
   // the window's parents and children as if the round does not stop in it
@@ -641,7 +645,7 @@ __global__ __launch_bounds__(1024) void k_select_chain(SArgs S) {
   }
   if (t == kSelChain - 1)
     while (!st.stop && top - st.consumed > 0)
-      select_window<KPER>(S, top, inc, s_p, s_w16, s_state, st);
+      select_window<kSelWin / 1024>(S, top, inc, s_p, s_w16, s_state, st);
   const bool done = st.stop || top - st.consumed <= 0;
   if (tid == 0) {
     if (!handed) hand_on(done);
@@ -721,7 +725,7 @@ __global__ __launch_bounds__(kExpandBlock) void k_expand(SArgs S, DevTables T, i
   // the chained select of the next round starts from cleared hand-offs
   // (this kernel runs after every select and before the next)
   if (blockIdx.x == 0) {
-    if (threadIdx.x < kSelChain * kLink) S.sel_link[threadIdx.x] = 0;
+    for (int i = threadIdx.x; i < kSelChain * kLink; i += kExpandBlock) S.sel_link[i] = 0;
     if (threadIdx.x == 0) S.ctrl->sel_ticket = 0;
   }
   // blocks past the round's parents leave before staging
