@@ -607,8 +607,10 @@ __global__ void k_tr_update(TrainArgs T, float* w, float* m, float* v, float* g,
     g[i] = gi;
   } else {
     const float beta1 = 0.9f, beta2 = 0.999f, eps = 1e-8f;
-    const float mi = beta1 * m[i] + (1.f - beta1) * gi;
-    const float vi = beta2 * v[i] + (1.f - beta2) * gi * gi;
+    // which product of a sum is fused is written out: left to the compiler, it
+    // changed with the code around it, and the weights' last bits with it
+    const float mi = fmaf(m[i], beta1, (1.f - beta1) * gi);
+    const float vi = fmaf(v[i], beta2, gi * ((1.f - beta2) * gi));
     m[i] = mi;
     v[i] = vi;
     const float wi = w[i] - lr * (mi / b1c) / (sqrtf(vi / b2c) + eps);
