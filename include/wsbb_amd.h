@@ -132,7 +132,10 @@ int wsbb_bound_batch_noalloc(wsbb_ctx *ctx, const uint8_t *permT,
                              const int32_t *l1, const int32_t *l2, int N,
                              int kind, int best, int32_t *out);
 /* Device-resident form: all pointers in HBM, asynchronous on the context's
- * stream (call wsbb_synchronize before reading d_out). */
+ * stream (call wsbb_synchronize before reading d_out).  That stream waits for
+ * no other: what another stream writes to the inputs has to be complete before
+ * the call.  The kernels check the limits: a node without -1 <= l1 < l2 <= n
+ * is left out, its d_out entry as it was. */
 int wsbb_bound_device(wsbb_ctx *ctx, const uint8_t *d_permT,
                       const int32_t *d_l1, const int32_t *d_l2, int N,
                       int kind, int32_t *d_out);

@@ -238,3 +238,39 @@ def test_host_batches_about_the_in_place_limit(kind):
             bad[n - 1, N - 1] = n
             with pytest.raises(wsbb_amd.WsbbError, match=f"index {n * N - 1}"):
                 eng.bound(bad, l1, l2, kind=kind)
+
+
+@pytest.mark.parametrize("n,m,scale", [(20, 5, 1), (50, 20, 1), (100, 3, 1), (20, 10, 9)])
+def test_device_batch_leaves_out_nodes_with_impossible_limits(n, m, scale):
+    """Limits in device memory that no node can have, among ordinary ones: the
+    kernels (matrix cores, both scans, LB1) leave those nodes out and bound the
+    others; times beyond a signed byte take the scan."""
+    p = scale * np.random.default_rng(n).integers(1, 100, size=(m, n)).astype(np.int32)
+    o = oracle.Oracle(p)
+    big = 2**31 - 1
+    wrong = [(-2, n), (-1, n + 1), (3, 3), (n, n), (5, 4), (n - 1, 0), (big, big), (-big - 1, big),
+             (big, -big - 1), (0, big), (-big, 1), (n + 40, n + 41)]
+    with wsbb_amd.Engine(p) as eng:
+        for N in (1, 200, 1025):
+            permT, l1, l2 = wsbb_amd.random_nodes(n, N, N)
+            at = np.random.default_rng(N).permutation(N)[:max(1, N // 3)]
+            ok = np.ones(N, bool)
+            ok[at] = False
+            b1, b2 = l1.copy(), l2.copy()
+            for i, k in enumerate(at):
+                b1[k], b2[k] = wrong[i % len(wrong)]
+            d = [eng.malloc(permT.nbytes)] + [eng.malloc(4 * N) for _ in range(3)]
+            for buf, a in zip(d, (permT, b1, b2)):
+                eng.h2d(buf, a)
+            for kind in (wsbb_amd.LB2, wsbb_amd.LB1):
+                ref = np.full(N, -7, np.int32)
+                ref[ok] = o.bound_batch(permT, l1, l2, kind=kind, threads=8)[ok]
+                for int16 in (1, 2):
+                    eng.set_int16(int16)
+                    eng.h2d(d[3], np.full(N, -7, np.int32))
+                    eng.bound_device(d[0], d[1], d[2], N, d[3], kind=kind)
+                    got = np.zeros(N, np.int32)
+                    eng.d2h(got, d[3])
+                    assert np.array_equal(got, ref), (N, kind, int16)
+            for buf in d:
+                eng.free(buf)

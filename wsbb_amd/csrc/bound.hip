@@ -238,7 +238,6 @@ __global__ __launch_bounds__(BLOCK) void bound_kernel(DevTables T, Src src, Boun
       l1 = -1;
       l2 = n;
     }
-    const int d1 = l1 + 1, d2 = n - l2;
     // children of a search round carry their parent's heads, tails and job
     // mask: a child extends them by the one or two jobs it places, and no
     // permutation is staged.  Otherwise the tile's first wave stages the
@@ -263,6 +262,13 @@ __global__ __launch_bounds__(BLOCK) void bound_kernel(DevTables T, Src src, Boun
           if (i0 + u < n) pl[(i0 + u) * bstride + tib * 64 + lane] = static_cast<uint8_t>(v[u]);
       }
     }
+    // after the staging, whose loads need not wait for the limits
+    if (!limits_ok(l1, l2, n)) {
+      valid = false;
+      l1 = -1;
+      l2 = n;
+    }
+    const int d1 = l1 + 1, d2 = n - l2;
     if (G > 1) __syncthreads();
 
     // heads of the prefix (set_tempsMachines_retardDebut 841-856) and tails
@@ -701,6 +707,11 @@ __global__ __launch_bounds__(256, (MM <= 20 ? 3 : 2)) void bound_kernel_pk(DevTa
           for (int u = 0; u < 16; ++u)
             if (i0 + u < n) pl[(i0 + u) * bst + tib * 128 + h * 64 + lane] = static_cast<uint8_t>(v[u]);
         }
+      }
+      if (!limits_ok(l1[h], l2[h], n)) {
+        valid[h] = false;
+        l1[h] = -1;
+        l2[h] = n;
       }
     }
     if (G > 1) __syncthreads();

@@ -192,6 +192,13 @@ __device__ __forceinline__ int perm_at(const uint8_t* col, int stride, int sw0,
   return col[static_cast<size_t>(src) * stride];
 }
 
+// Limits a node can have.  The host checks those it is given; a batch resident
+// in device memory is checked by the kernels, which leave any other node out:
+// its limits would run the recurrences and a block's sort past their arrays.
+__device__ __forceinline__ bool limits_ok(int l1, int l2, int n) {
+  return l1 >= -1 && l1 < l2 && l2 <= n;
+}
+
 // Node source: explicit position-major nodes.
 struct BatchSource {
   static constexpr bool kState = false;  // no parent state: heads/tails from the permutation

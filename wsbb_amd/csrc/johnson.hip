@@ -279,10 +279,12 @@ __global__ __launch_bounds__(256, (NB == 2 && KB <= 2 ? 3 : 2)) void k_johnson(D
 
   // lane l answers for nodes tile0 + 64 r + l
   int l1[RUNS], l2[RUNS];
+  bool live[RUNS];
 #pragma unroll
   for (int r = 0; r < RUNS; ++r) {
     l1[r] = -1;
     l2[r] = n;
+    live[r] = tile0 + 64 * r + lane < N;
   }
   // the wave's runs of prefixes and of suffixes (none: -1); run q covers 64
   // of the block's nodes
@@ -341,6 +343,11 @@ __global__ __launch_bounds__(256, (NB == 2 && KB <= 2 ? 3 : 2)) void k_johnson(D
 #pragma unroll
           for (int u = 0; u < 16; ++u)
             if (i0 + u < n) pl[(i0 + u) * TN] = static_cast<uint8_t>(v[u]);
+        }
+        if (!limits_ok(a1, a2, n)) {
+          live[r] = false;
+          l1[r] = -1;
+          l2[r] = n;
         }
       }
     }
@@ -741,7 +748,7 @@ __global__ __launch_bounds__(256, (NB == 2 && KB <= 2 ? 3 : 2)) void k_johnson(D
       if (wi == 0)
         for (int k = 1; k < W; ++k) res = max(res, comb[(wave + k) * TN + mine_l]);
     }
-    if (wi == 0 && node < N) A.out[H.list ? H.list[node] : node] = res;
+    if (wi == 0 && live[r]) A.out[H.list ? H.list[node] : node] = res;
   }
 }
 
