@@ -168,8 +168,10 @@ int wsbb_timer_stop(wsbb_ctx *ctx, float *ms);
  * groups: waves that split the pairs of one 64-node tile (1, 2, 4, 8 or
  * 16; 8 and 16 apply to plain LB2 with at most 16 machines, else 4);
  * grid_blocks: cap on 256-thread blocks (0 = automatic).  wsbb_autotune
- * times every shape on a synthetic batch of N nodes and keeps the fastest
- * for batches of that size class; shapes/times are written if non-NULL. */
+ * times every shape that differs for the instance's LB2 kernel (at most 15)
+ * on a synthetic batch of N nodes and keeps the fastest for that kernel's
+ * batches of that size class, search rounds excepted; shapes (groups,
+ * grid_blocks) and times are written if non-NULL. */
 int wsbb_set_launch(wsbb_ctx *ctx, int groups, int grid_blocks);
 int wsbb_autotune(wsbb_ctx *ctx, int N, int reps, int32_t *shapes,
                   float *ms, int *count);

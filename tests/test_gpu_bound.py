@@ -274,3 +274,23 @@ def test_device_batch_leaves_out_nodes_with_impossible_limits(n, m, scale):
                     assert np.array_equal(got, ref), (N, kind, int16)
             for buf in d:
                 eng.free(buf)
+
+
+@pytest.mark.parametrize("n,m,scale,groups", [(20, 24, 1, [1, 2, 4]), (50, 5, 1, [1, 2]), (100, 5, 1, [1]),
+                                              (20, 20, 9, [1, 2, 4]), (20, 5, 9, [1, 2, 4, 8, 16])])
+def test_autotune_times_the_shapes_it_lists(n, m, scale, groups):
+    """Every shape once: the waves that can split a tile's pairs, under each
+    grid only for the scans (times beyond a signed byte), whose blocks loop."""
+    p = scale * np.random.default_rng(n).integers(1, 100, size=(m, n)).astype(np.int32)
+    permT, l1, l2 = wsbb_amd.random_nodes(n, 2000, 1)
+    ref = oracle.Oracle(p).bound_batch(permT, l1, l2, threads=8)
+    with wsbb_amd.Engine(p) as eng:
+        for _ in range(2):  # the second finds the first's choice in place
+            shapes = eng.autotune(2000, reps=50)
+            assert len(set(s[:2] for s in shapes)) == len(shapes)
+            assert sorted(set(s[0] for s in shapes)) == groups
+            assert len(set(s[1] for s in shapes)) == (1 if scale == 1 else 3)
+            ms = {s[0]: s[2] for s in shapes}
+            if n == 20 and scale == 1:  # 32 tiles of 276 pairs: one wave a tile is what it says
+                assert ms[1] > 1.2 * ms[4], ms
+            assert np.array_equal(eng.bound(permT, l1, l2), ref)

@@ -77,10 +77,8 @@ static bool johnson_fits(const Instance& I) {
 
 int wsbb_ctx::groups_for(int N) const {
   if (launch.groups > 1) return launch.groups;
-  const int tiles = (N + 63) / 64;
-  int cls = 0;
-  while ((1 << (cls + 1)) <= tiles && cls < 31) ++cls;
-  if (tuned_groups[cls] > 0) return tuned_groups[cls];
+  const int tiles = (N + 63) / 64, tuned = tuned_groups[size_class(N)];
+  if (tuned > 0) return tuned;
   // enough wavefronts to give every SIMD of every CU at least one
   const int want = num_cus * 4;
   if (tiles >= want) return 1;
@@ -185,6 +183,7 @@ int wsbb_create(const int32_t* p, int n, int m, int device, wsbb_ctx** out) {
   // the instance is checked (host only) before any device is touched
   auto* ctx = new wsbb_ctx();
   for (int& g : ctx->tuned_groups) g = -1;
+  for (int& g : ctx->tuned_waves) g = -1;
   std::string err = ctx->inst.build(p, n, m);
   if (!err.empty()) {
     set_error(err);
@@ -436,7 +435,7 @@ int wsbb_bound_batch_ex(wsbb_ctx* ctx, const uint8_t* permT, const int32_t* l1,
   A.best = best;
   A.groups = ctx->groups_for(N);
   A.pk = ctx->int16_for(N);
-  ctx->johnson_args(A);
+  ctx->johnson_batch_args(A);
   A.out = reinterpret_cast<int32_t*>(base + o_out);
   A.argmax = argmax ? reinterpret_cast<int32_t*>(base + o_am) : nullptr;
   A.pairv = pairv ? reinterpret_cast<int32_t*>(base + o_pv) : nullptr;
@@ -552,7 +551,7 @@ int wsbb_bound_batch_noalloc(wsbb_ctx* ctx, const uint8_t* permT, const int32_t*
   A.best = best;
   A.groups = ctx->groups_for(N);
   A.pk = ctx->int16_for(N);
-  ctx->johnson_args(A);
+  ctx->johnson_batch_args(A);
   A.out = reinterpret_cast<int32_t*>(base + o_out);
   WSBB_HIP(launch_bound(ctx->T, src, A, ctx->grid_cap(), st), "bound kernel launch");
   WSBB_HIP(hipMemcpyAsync(out, A.out, size_t(4) * N, hipMemcpyDeviceToHost, st), "D2H out");
@@ -574,7 +573,7 @@ int wsbb_bound_device(wsbb_ctx* ctx, const uint8_t* d_permT, const int32_t* d_l1
   A.best = -1;
   A.groups = ctx->groups_for(N);
   A.pk = ctx->int16_for(N);
-  ctx->johnson_args(A);
+  ctx->johnson_batch_args(A);
   A.out = d_out;
   WSBB_HIP(launch_bound(ctx->T, src, A, ctx->grid_cap(), ctx->stream), "bound kernel launch");
   return WSBB_OK;
@@ -682,10 +681,15 @@ int wsbb_autotune(wsbb_ctx* ctx, int N, int reps, int32_t* shapes, float* ms,
   (void)hipMemcpy(dp, permT.data(), permT.size(), hipMemcpyHostToDevice);
   (void)hipMemcpy(d1, l1.data(), 4 * size_t(N), hipMemcpyHostToDevice);
   (void)hipMemcpy(d2, l2.data(), 4 * size_t(N), hipMemcpyHostToDevice);
-  // 8 and 16 waves per tile run in 1024-thread blocks (up to 16 machines)
+  // distinct shapes only: the matrix-core form splits a tile's pairs over as
+  // many waves as its row tiles leave of four, and its blocks do not loop, so
+  // a smaller grid is the same work in more launches; of the scans, 8 and 16
+  // waves per tile run in 1024-thread blocks (up to 16 machines)
+  const bool mfma = ctx->mfma_for() != 0;
   const int cand_groups[5] = {1, 2, 4, 8, 16};
-  const int n_groups = ctx->T.m <= 16 ? 5 : 3;
-  const int cand_grid[3] = {ctx->num_cus * 4, ctx->num_cus * 8, ctx->num_cus * 16};
+  const int n_groups = mfma ? johnson_splits(n) : ctx->T.m <= 16 ? 5 : 3;
+  std::vector<int> cand_grid = {ctx->num_cus * 4, ctx->num_cus * 8, ctx->num_cus * 16};
+  if (mfma) cand_grid = {ctx->num_cus * 16};
   int best_g = 1, best_grid = 0, idx = 0;
   float best_t = 1e30f;
   const Launch saved = ctx->launch;
@@ -702,7 +706,8 @@ int wsbb_autotune(wsbb_ctx* ctx, int N, int reps, int32_t* shapes, float* ms,
       A.best = -1;
       A.groups = g;
       A.pk = ctx->int16_for(N);
-  ctx->johnson_args(A);
+      ctx->johnson_args(A);
+      A.waves = g;  // one too is asked for, not left to the launch
       A.out = static_cast<int32_t*>(dout);
       hipError_t e = launch_bound(ctx->T, src, A, grid, ctx->stream);  // warm-up
       if (e == hipSuccess) e = hipEventRecord(ctx->ev_start, ctx->stream);
@@ -733,11 +738,13 @@ int wsbb_autotune(wsbb_ctx* ctx, int N, int reps, int32_t* shapes, float* ms,
   ctx->launch = saved;
   if (rc != WSBB_OK) return rc;
   if (count) *count = idx;
-  const int tiles = (N + 63) / 64;
-  int cls = 0;
-  while ((1 << (cls + 1)) <= tiles && cls < 31) ++cls;
-  ctx->tuned_groups[cls] = best_g;
-  if (ctx->launch.grid_cap == 0) ctx->launch.grid_cap = best_grid;
+  const int cls = wsbb_ctx::size_class(N);
+  if (mfma) {
+    ctx->tuned_waves[cls] = best_g;
+  } else {
+    ctx->tuned_groups[cls] = best_g;
+    if (ctx->launch.grid_cap == 0) ctx->launch.grid_cap = best_grid;
+  }
   return WSBB_OK;
 }
 

@@ -101,8 +101,9 @@ struct wsbb_ctx {
   int rounds_per_sync = 4;       // rounds queued between host status checks
   wsbb_trace_fn trace_fn = nullptr;  // per-round search trace (one round per sync)
   void* trace_user = nullptr;
-  // autotuned shapes by batch size class (log2 of tiles), -1 = not tuned
-  int tuned_groups[32];
+  // autotuned shapes by batch size class (log2 of tiles), -1 = not tuned: of
+  // the scans, and of the matrix-core form
+  int tuned_groups[32], tuned_waves[32];
   wsbb::SearchState* search = nullptr;
   wsbb::SelectorState* selector = nullptr;
 
@@ -114,12 +115,25 @@ struct wsbb_ctx {
   // the matrix cores bound faster than either scan at every batch size; a
   // caller who asks for the int16 form gets it
   int mfma_for() const { return T.mf != nullptr && launch.int16 != 2; }
+  static int size_class(int N) {
+    const int tiles = (N + 63) / 64;
+    int cls = 0;
+    while ((1 << (cls + 1)) <= tiles && cls < 31) ++cls;
+    return cls;
+  }
+  // the split a caller asked for, or the launch's own
   void johnson_args(wsbb::BoundArgs& A) const {
     A.mfma = mfma_for();
     A.num_cus = num_cus;
-    int tiles = (A.N + 63) / 64, cls = 0;  // as groups_for
-    while ((1 << (cls + 1)) <= tiles && cls < 31) ++cls;
-    A.waves = launch.groups > 1 ? launch.groups : tuned_groups[cls] > 0 ? tuned_groups[cls] : 0;
+    A.waves = launch.groups > 1 ? launch.groups : 0;
+  }
+  // the same for a batch of A.N nodes, with the tuned split of its size.  A
+  // search round is not one: A.N is its capacity, and its live children,
+  // often far fewer, are not the batch that was tuned.
+  void johnson_batch_args(wsbb::BoundArgs& A) const {
+    johnson_args(A);
+    const int tuned = tuned_waves[size_class(A.N)];
+    if (A.waves == 0 && tuned > 0) A.waves = tuned;
   }
   // two nodes per lane pays once a batch gives every SIMD two 128-node tiles;
   // smaller launches are latency-bound and prefer more wavefronts

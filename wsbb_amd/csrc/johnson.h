@@ -47,6 +47,8 @@ struct JohnsonShape {
 // The layout for N nodes; waves: ways to split the pairs, or 0 (chosen).
 JohnsonShape johnson_shape(int n, int P, int N, int waves, bool subset, int num_cus);
 inline int johnson_block_nodes(const JohnsonShape& H) { return (H.wide ? 128 : 64) * H.tpb; }
+// How many of 1, 2 and 4 waves can split the pairs of one tile of n jobs.
+inline int johnson_splits(int n) { return n <= 32 ? 3 : n <= 64 ? 2 : 1; }
 // Instances of one class share a kernel: equal padded machines, row tiles and
 // column blocks.
 int johnson_class(int n, int m);
