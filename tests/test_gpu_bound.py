@@ -294,3 +294,38 @@ def test_autotune_times_the_shapes_it_lists(n, m, scale, groups):
             if n == 20 and scale == 1:  # 32 tiles of 276 pairs: one wave a tile is what it says
                 assert ms[1] > 1.2 * ms[4], ms
             assert np.array_equal(eng.bound(permT, l1, l2), ref)
+
+
+def device_us(eng, permT, l1, l2, reps=10):
+    """Bounds of a resident batch and the least of five timings of a pass."""
+    N = l1.shape[0]
+    d = [eng.malloc(permT.nbytes)] + [eng.malloc(4 * N) for _ in range(3)]
+    for buf, a in zip(d, (permT, l1, l2)):
+        eng.h2d(buf, a)
+    eng.bound_device(d[0], d[1], d[2], N, d[3])
+    times = []
+    for _ in range(5):
+        eng.timer_start()
+        for _ in range(reps):
+            eng.bound_device(d[0], d[1], d[2], N, d[3])
+        times.append(eng.timer_stop() / reps * 1e3)
+    out = np.zeros(N, np.int32)
+    eng.d2h(out, d[3])
+    for buf in d:
+        eng.free(buf)
+    return out, min(times)
+
+
+def test_large_batches_about_32_jobs():
+    """31 and 32 jobs have one row tile, as 30, and two column blocks: their
+    large batches stay on 64-node tiles, and cost little more."""
+    N, us = 300_001, {}
+    for n in (30, 31, 32):
+        p = np.random.default_rng(n).integers(1, 100, size=(20, n)).astype(np.int32)
+        permT, l1, l2 = wsbb_amd.random_nodes(n, N, n)
+        with wsbb_amd.Engine(p) as eng:
+            out, us[n] = device_us(eng, permT, l1, l2)
+        idx = np.r_[0:300, N - 300:N, np.random.default_rng(1).choice(N, 2000, replace=False)]
+        assert np.array_equal(out[idx], oracle.Oracle(p).bound_batch(permT[:, idx], l1[idx], l2[idx], threads=8))
+    # 97, 113 and 115 us; on 128-node tiles 179 and 182
+    assert max(us[31], us[32]) < 1.4 * us[30], us

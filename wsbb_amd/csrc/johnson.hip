@@ -846,12 +846,14 @@ JohnsonShape johnson_shape(int n, int P, int N, int waves, bool subset, int num_
                                                      : 1;
   H.groups = subset ? 1 : std::max(1, std::min(H.groups, 4 / H.rts));
   // Tiles of 128 nodes halve the fragments' way through the L1 and the scalar
-  // work, for twice the registers: with two column blocks of jobs and more,
-  // from two waves per SIMD on (us for 64 / 128 nodes: 50x20, 65 536 nodes 56
-  // / 66; 130 000 nodes 101 / 93; 2^20 nodes 654 / 600; 100x10, 65 521 nodes
-  // 70 / 55).  With one, the start clocks and tails of 128 nodes leave room
-  // in LDS for one wave per SIMD (20x20, 300 000 nodes: 83 / 151).
-  H.wide = !subset && column_blocks(n) >= 2 && H.groups == 1 &&
+  // work, for twice the registers: with two row tiles of jobs and more, from
+  // two waves per SIMD on (us for 64 / 128 nodes: 50x20, 65 536 nodes 56 / 66;
+  // 130 000 nodes 101 / 93; 2^20 nodes 654 / 600; 100x10, 65 521 nodes 70 /
+  // 55).  With one row tile a block holds four such tiles, whose start clocks
+  // and tails leave room in LDS for one wave per SIMD: 300 000 nodes, 20x20 83
+  // / 151, 32x20 115 / 182, 32x5 30 / 40; 2^20 nodes, 32x20 332 / 485, 32x5 79
+  // / 88 (at 262 017 nodes, whose blocks just fill the chip, 32x5 is 28 / 25).
+  H.wide = !subset && H.rts >= 2 && H.groups == 1 &&
            static_cast<long long>((N + 127) / 128) * H.rts >= 2 * simds;
   H.tpb = std::max(1, 4 / (H.rts * H.groups));
   return H;
