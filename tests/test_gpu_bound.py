@@ -329,3 +329,18 @@ def test_large_batches_about_32_jobs():
         assert np.array_equal(out[idx], oracle.Oracle(p).bound_batch(permT[:, idx], l1[idx], l2[idx], threads=8))
     # 97, 113 and 115 us; on 128-node tiles 179 and 182
     assert max(us[31], us[32]) < 1.4 * us[30], us
+
+
+def test_large_batches_of_three_row_tiles():
+    """65 to 94 jobs: large batches stay on 64-node tiles, and 90 jobs cost no
+    more than 100, which fill a block's four waves."""
+    N, us = 300_001, {}
+    for n in (65, 90, 94, 100):
+        p = np.random.default_rng(n).integers(1, 100, size=(5, n)).astype(np.int32)
+        permT, l1, l2 = wsbb_amd.random_nodes(n, N, n)
+        with wsbb_amd.Engine(p) as eng:
+            out, us[n] = device_us(eng, permT, l1, l2)
+        idx = np.r_[0:300, N - 300:N, np.random.default_rng(1).choice(N, 2000, replace=False)]
+        assert np.array_equal(out[idx], oracle.Oracle(p).bound_batch(permT[:, idx], l1[idx], l2[idx], threads=8))
+    # 123 and 137 us; on 128-node tiles 90 jobs take 165
+    assert us[90] < 1.05 * us[100], us

@@ -853,7 +853,14 @@ JohnsonShape johnson_shape(int n, int P, int N, int waves, bool subset, int num_
   // and tails leave room in LDS for one wave per SIMD: 300 000 nodes, 20x20 83
   // / 151, 32x20 115 / 182, 32x5 30 / 40; 2^20 nodes, 32x20 332 / 485, 32x5 79
   // / 88 (at 262 017 nodes, whose blocks just fill the chip, 32x5 is 28 / 25).
-  H.wide = !subset && H.rts >= 2 && H.groups == 1 &&
+  // With three row tiles a block is one tile of three waves, two of which run
+  // its prefixes and then its suffixes while the third waits: 90 jobs, 131 072
+  // nodes, 5 machines 56 / 72, 20 machines 220 / 244; 2^20 nodes, 5 machines
+  // 380 / 520, 10 machines 600 / 787 (95 and 96 jobs, whose fourth column
+  // block holds the constants, have two waves per SIMD at 64 nodes too: 96
+  // jobs, 2^20 nodes, 5 machines 629 / 557, 10 machines 953 / 863).
+  const bool third_idle = H.rts == 3 && column_blocks(n) == 3;
+  H.wide = !subset && H.rts >= 2 && !third_idle && H.groups == 1 &&
            static_cast<long long>((N + 127) / 128) * H.rts >= 2 * simds;
   H.tpb = std::max(1, 4 / (H.rts * H.groups));
   return H;
