@@ -344,3 +344,29 @@ def test_large_batches_of_three_row_tiles():
         assert np.array_equal(out[idx], oracle.Oracle(p).bound_batch(permT[:, idx], l1[idx], l2[idx], threads=8))
     # 123 and 137 us; on 128-node tiles 90 jobs take 165
     assert us[90] < 1.05 * us[100], us
+
+
+@pytest.mark.parametrize("n,m,N,faster", [
+    # the scans' side and the matrix cores' at the rule's sizes, pairs and jobs
+    (11, 3, 98_303, False), (11, 3, 98_304, False), (11, 4, 262_143, False), (11, 3, 262_144, False),
+    (8, 4, 300_001, True), (5, 2, 524_288, True), (11, 3, 1 << 20, True), (11, 6, 1 << 20, False),
+    (33, 3, 1 << 20, True), (65, 3, 1 << 20, True), (96, 5, 1 << 20, True), (97, 3, 300_001, False),
+    (21, 2, 524_287, False), (31, 3, 1 << 20, False), (8, 3, 49_152, False), (95, 5, 200_001, True)])
+def test_large_batches_of_few_pairs(n, m, N, faster):
+    """Both forms of plain LB2 on the same resident batch, against the oracle
+    on a sample; where the rule's measurements say that the scans are clearly
+    faster (by 12% and more), the call is as fast as they are."""
+    p = np.random.default_rng(100 * n + m).integers(1, 100, size=(m, n)).astype(np.int32)
+    permT, l1, l2 = wsbb_amd.random_nodes(n, N, 3)
+    idx = np.r_[0:300, N - 300:N, np.random.default_rng(1).choice(N, 3000, replace=False)]
+    ref = oracle.Oracle(p).bound_batch(permT[:, idx], l1[idx], l2[idx], threads=8)
+    with wsbb_amd.Engine(p) as eng:
+        out, us = device_us(eng, permT, l1, l2)
+        eng.set_int16(2)
+        scan, scan_us = device_us(eng, permT, l1, l2)
+        eng.set_int16(0)
+        other, _ = device_us(eng, permT, l1, l2, reps=1)
+    assert np.array_equal(out[idx], ref)
+    assert np.array_equal(out, scan) and np.array_equal(out, other)
+    if faster:
+        assert us < 1.07 * scan_us, (us, scan_us)

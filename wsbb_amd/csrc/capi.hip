@@ -685,7 +685,7 @@ int wsbb_autotune(wsbb_ctx* ctx, int N, int reps, int32_t* shapes, float* ms,
   // many waves as its row tiles leave of four, and its blocks do not loop, so
   // a smaller grid is the same work in more launches; of the scans, 8 and 16
   // waves per tile run in 1024-thread blocks (up to 16 machines)
-  const bool mfma = ctx->mfma_for() != 0;
+  const bool mfma = ctx->mfma_for() && !ctx->few_pairs(N);
   const int cand_groups[5] = {1, 2, 4, 8, 16};
   const int n_groups = mfma ? johnson_splits(n) : ctx->T.m <= 16 ? 5 : 3;
   std::vector<int> cand_grid = {ctx->num_cus * 4, ctx->num_cus * 8, ctx->num_cus * 16};
@@ -707,6 +707,7 @@ int wsbb_autotune(wsbb_ctx* ctx, int N, int reps, int32_t* shapes, float* ms,
       A.groups = g;
       A.pk = ctx->int16_for(N);
       ctx->johnson_args(A);
+      A.mfma = mfma;
       A.waves = g;  // one too is asked for, not left to the launch
       A.out = static_cast<int32_t*>(dout);
       hipError_t e = launch_bound(ctx->T, src, A, grid, ctx->stream);  // warm-up

@@ -112,9 +112,34 @@ struct wsbb_ctx {
     return num_cus * 16;  // 16 blocks per CU: a 2^20-node batch, one per four tiles
   }
   int groups_for(int N) const;
-  // the matrix cores bound faster than either scan at every batch size; a
-  // caller who asks for the int16 form gets it
+  // a caller who asks for the int16 form gets it
   int mfma_for() const { return T.mf != nullptr && launch.int16 != 2; }
+  // A large batch of few pairs is nearly all heads and tails, which the scans
+  // run with less work (from 2^18 nodes on two nodes a lane), while a pair
+  // costs the matrix cores whole tiles: the scans are faster where pairs x
+  // jobs is small against the jobs that the tiles leave empty, counted from
+  // the sizes at which they stop to be (20 and 29 of one row tile, 56 of two,
+  // 116 of three; 230 at 95 and 96 jobs, whose fourth column block costs the
+  // kernel a wave per SIMD).  With more than 96 jobs a block's four waves
+  // share heads and tails, and the matrix cores win.  us, scan / matrix cores:
+  // 2^20 nodes, 11 jobs 3 machines 33 / 41, 5 machines 44 / 47, 6 machines 52 /
+  // 52; 33 jobs 4 machines 105 / 123, 6 machines 146 / 143; 65 jobs 5 machines
+  // 290 / 321, 6 machines 355 / 347; 90 jobs 3 machines 294 / 347, 5 machines
+  // 421 / 380; 96 jobs 5 machines 446 / 556; 100 jobs 3 machines 389 / 361.
+  // 300 000 nodes, 11 jobs 3 machines 17 / 18, 4 machines 19 / 19; 65 jobs 3
+  // machines 90 / 93, 5 machines 130 / 104.  131 072 nodes, 11 jobs 3 machines
+  // 10.1 / 10.4, 96 jobs 5 machines 73 / 78.  65 536 nodes, 8 jobs 3 machines
+  // 7.4 / 8.1, 33 jobs 3 machines 16 / 12, 96 jobs 3 machines 41 / 40.
+  bool few_pairs(int N) const {
+    const int n = T.n, P = T.P, simds = 4 * num_cus;
+    if (n > 96) return false;
+    const int empty = (n <= 20 ? 20 : n <= 32 ? 29 : n <= 64 ? 56 : n <= 94 ? 116 : 230) - n;
+    if (N >= 256 * simds) {
+      if (T.steps16 == nullptr || !int16_for(N)) return false;
+      return N >= 512 * simds ? P <= 28 && P * n < 14 * empty : 2 * P * n <= 9 * empty;
+    }
+    return N >= (n <= 10 ? 48 : 96) * simds && (n > 94 ? P <= 10 : P <= 3 && 2 * P * n <= 9 * empty);
+  }
   static int size_class(int N) {
     const int tiles = (N + 63) / 64;
     int cls = 0;
@@ -132,6 +157,7 @@ struct wsbb_ctx {
   // often far fewer, are not the batch that was tuned.
   void johnson_batch_args(wsbb::BoundArgs& A) const {
     johnson_args(A);
+    A.mfma = A.mfma && !few_pairs(A.N);
     const int tuned = tuned_waves[size_class(A.N)];
     if (A.waves == 0 && tuned > 0) A.waves = tuned;
   }
