@@ -97,7 +97,11 @@ int wsbb_info(const wsbb_ctx *ctx, int *n, int *m, int *pairs, int *num_cus);
  * best != -1 the first running maximum above best, 154-161) or LB1.
  * Replaces the H2D copy + Evaluate_ON_GPU + D2H of gpu::decompose_on_cpu
  * (src/gpu.cu:211-234; kernel src/bound_flowshop_gpu.cu:619-674).
- * Host-buffer form: copies in, bounds, copies out, synchronises. */
+ * Host-buffer form: copies in, bounds, copies out, synchronises.  Nodes and
+ * bounds of up to 1 MiB go through a pinned buffer of that size that the
+ * library holds for each GPU from the first wsbb_create on it until the
+ * process ends (a call made while another thread's is using it: through one
+ * of its context's own). */
 int wsbb_bound_batch(wsbb_ctx *ctx, const uint8_t *permT, const int32_t *l1,
                      const int32_t *l2, int N, int kind, int best,
                      int32_t *out);

@@ -370,3 +370,52 @@ def test_large_batches_of_few_pairs(n, m, N, faster):
     assert np.array_equal(out, scan) and np.array_equal(out, other)
     if faster:
         assert us < 1.07 * scan_us, (us, scan_us)
+
+
+def test_first_small_batch_of_an_engine_allocates_no_staging():
+    """A new engine's first 64-node call costs about what its next ones do
+    (the pinned staging is the device's); making staging for it took as long
+    again as the call."""
+    import time
+
+    p = oracle.taillard(1)[3]
+    nodes = wsbb_amd.random_nodes(20, 64, 1)
+    ref = oracle.Oracle(p).bound_batch(*nodes)
+    first, later = [], []
+    for _ in range(41):
+        with wsbb_amd.Engine(p) as eng:
+            eng.synchronize()
+            for times in (first, later):
+                t = time.perf_counter()
+                got = eng.bound(*nodes)
+                times.append(time.perf_counter() - t)
+                assert np.array_equal(got, ref)
+    assert np.median(first) < 1.5 * np.median(later), (np.median(first), np.median(later))
+
+
+def test_small_batches_of_engines_on_threads():
+    """Calls of several threads' engines overlap: one stages in the device's
+    buffer, the others in their own."""
+    import threading
+
+    ps = [oracle.taillard(t)[3] for t in (1, 11, 21, 51)]
+    wrong = []
+
+    def work(i):
+        p = ps[i]
+        n = p.shape[1]
+        with wsbb_amd.Engine(p) as eng:
+            for rep in range(60):
+                N = (1, 64, 4096, 15000)[(i + rep) % 4]
+                permT, l1, l2 = wsbb_amd.random_nodes(n, N, 10 * i + rep)
+                pick = np.unique(np.r_[0:min(N, 40), max(0, N - 40):N])
+                want = oracle.Oracle(p).bound_batch(permT[:, pick], l1[pick], l2[pick])
+                if not np.array_equal(eng.bound(permT, l1, l2)[pick], want):
+                    wrong.append((i, rep, N))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong

@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <vector>
 
@@ -38,6 +39,46 @@ static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 static std::mutex g_scratch_mu;
 static uint8_t* g_scratch_ptr[kMaxDevices] = {};
 
+// Pinned staging of small host batches, made with the array's address and kept
+// as long.  One a context was made in its first such call and freed with it:
+// 20x5, 64 nodes, a context's first call 49 us against 24, its end 67 against
+// 53.  A call leases the buffer; one that finds it leased (another thread's
+// context on the same device) stages in its context's own.
+constexpr size_t kPinnedBytes = size_t(1) << 20;
+static HostBuf g_pinned[kMaxDevices];
+static bool g_pinned_leased[kMaxDevices] = {};
+
+class PinnedLease {
+ public:
+  explicit PinnedLease(wsbb_ctx* ctx) : device_(ctx->device), stream_(ctx->stream) {
+    {
+      std::lock_guard<std::mutex> lock(g_scratch_mu);
+      if (g_pinned[device_].ptr && !g_pinned_leased[device_]) {
+        g_pinned_leased[device_] = shared_ = true;
+        buf_ = &g_pinned[device_];
+      }
+    }
+    if (!shared_ && ctx->pinned.reserve(kPinnedBytes)) buf_ = &ctx->pinned;
+  }
+  // a call that failed half way may have left a kernel on the buffer
+  ~PinnedLease() {
+    if (!shared_) return;
+    if (in_flight) (void)hipStreamSynchronize(stream_);
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    g_pinned_leased[device_] = false;
+  }
+  PinnedLease(const PinnedLease&) = delete;
+  PinnedLease& operator=(const PinnedLease&) = delete;
+  const HostBuf* get() const { return buf_; }  // null: no pinned memory to be had
+  bool in_flight = false;
+
+ private:
+  int device_;
+  hipStream_t stream_;
+  const HostBuf* buf_ = nullptr;
+  bool shared_ = false;
+};
+
 // with `device` current: resolve that device's copy of the array once
 static int scratch_setup(int device) {
   std::lock_guard<std::mutex> lock(g_scratch_mu);
@@ -50,6 +91,7 @@ static int scratch_setup(int device) {
   const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
   if (e != hipSuccess) return hip_fail(e, "hipGetSymbolAddress(scratch)");
   g_scratch_ptr[device] = static_cast<uint8_t*>(ptr);
+  (void)g_pinned[device].reserve(kPinnedBytes);  // without it contexts make their own
   return WSBB_OK;
 }
 
@@ -352,7 +394,7 @@ int wsbb_info(const wsbb_ctx* ctx, int* n, int* m, int* pairs, int* num_cus) {
   return WSBB_OK;
 }
 
-// Plain host batches up to this size are copied by the host into pinned memory
+// Plain host batches up to kPinnedBytes are copied by the host into pinned memory
 // that the kernel reads and writes in place: every node is read once, so the
 // transfer is the kernel's own loads, and a call is one launch and one wait.
 // Above it copies into device memory win (their transfer runs ahead of the
@@ -360,7 +402,6 @@ int wsbb_info(const wsbb_ctx* ctx, int* n, int* m, int* pairs, int* num_cus) {
 // nodes 23.7 / 39.8, 20x10 4096 31.8 / 49.4, 30000 (0.96 MB) 88 / 99, 60000
 // 163 / 159, 50x20 14000 (0.87 MB) 108 / 113, 60000 360 / 272.  (Copied, and
 // with the argument checks below leaving at the first fault: 49.9 and 74.6.)
-constexpr size_t kPinnedBytes = size_t(1) << 20;
 
 // Whole passes without an exit (which the compiler vectorises); the first
 // offender is looked for only when there is one.
@@ -410,14 +451,16 @@ int wsbb_bound_batch_ex(wsbb_ctx* ctx, const uint8_t* permT, const int32_t* l1,
   const size_t total = o_feat + (feat ? al(size_t(4) * 5 * m * N) : 0);
   WSBB_HIP(hipSetDevice(ctx->device), "hipSetDevice");
   hipStream_t st = ctx->stream;
-  const bool pinned = !argmax && !pairv && !sel && !feat && total <= kPinnedBytes &&
-                      ctx->pinned.reserve(kPinnedBytes);  // whole: an allocation costs 40 us at any size
+  std::optional<PinnedLease> lease;
+  if (!argmax && !pairv && !sel && !feat && total <= kPinnedBytes) lease.emplace(ctx);
+  const HostBuf* pinned = lease ? lease->get() : nullptr;
   char* base;  // of the nodes and results, as the kernel sees them
   if (pinned) {
-    base = ctx->pinned.dev;
-    memcpy(ctx->pinned.ptr + o_perm, permT, size_t(n) * N);
-    memcpy(ctx->pinned.ptr + o_l1, l1, size_t(4) * N);
-    memcpy(ctx->pinned.ptr + o_l2, l2, size_t(4) * N);
+    base = pinned->dev;
+    memcpy(pinned->ptr + o_perm, permT, size_t(n) * N);
+    memcpy(pinned->ptr + o_l1, l1, size_t(4) * N);
+    memcpy(pinned->ptr + o_l2, l2, size_t(4) * N);
+    lease->in_flight = true;
   } else {
     WSBB_HIP(ctx->batch.reserve(total), "hipMalloc(batch)");
     base = ctx->batch.as<char>();
@@ -445,7 +488,8 @@ int wsbb_bound_batch_ex(wsbb_ctx* ctx, const uint8_t* permT, const int32_t* l1,
   WSBB_HIP(launch_bound(ctx->T, src, A, ctx->grid_cap(), st), "bound kernel launch");
   if (pinned) {
     WSBB_HIP(hipStreamSynchronize(st), "hipStreamSynchronize");
-    memcpy(out, ctx->pinned.ptr + o_out, size_t(4) * N);
+    lease->in_flight = false;
+    memcpy(out, pinned->ptr + o_out, size_t(4) * N);
     return WSBB_OK;
   }
   WSBB_HIP(hipMemcpyAsync(out, A.out, size_t(4) * N, hipMemcpyDeviceToHost, st), "D2H out");

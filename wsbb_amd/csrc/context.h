@@ -41,7 +41,7 @@ struct DevBuf {
   }
 };
 
-// Grow-only pinned host memory that kernels read and write in place.
+// Pinned host memory that kernels read and write in place.
 struct HostBuf {
   char* ptr = nullptr;  // as the host sees it
   char* dev = nullptr;  // as kernels do
@@ -93,7 +93,7 @@ struct wsbb_ctx {
   wsbb::DevTables T{};
   wsbb::DevBuf tables;  // every instance table in one allocation
   wsbb::DevBuf batch;   // staging for host-buffer batch calls
-  wsbb::HostBuf pinned; // and for the small ones
+  wsbb::HostBuf pinned; // and for small ones while another call holds the device's
   wsbb::Launch launch;
   int pool_capacity = 1 << 24;  // device node-pool capacity (nodes)
   int profile_every = 0;         // time every k-th round's bound launch in wsbb_solve
