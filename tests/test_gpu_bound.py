@@ -419,3 +419,18 @@ def test_small_batches_of_engines_on_threads():
     for t in threads:
         t.join()
     assert not wrong
+
+
+@pytest.mark.parametrize("n", [31, 32, 33, 62, 64, 65, 94, 96, 97])
+@pytest.mark.parametrize("m", [8, 16, 24])
+def test_lb2_large_batches_at_operand_edges(n, m):
+    """Batches large enough for one wave a row tile (every size) and for
+    128-node tiles (two row tiles, three with four column blocks, four) at
+    the edges of the operands, the last tile partial."""
+    N = 131_137
+    p = np.random.default_rng(n * m).integers(0, 128, size=(m, n)).astype(np.int32)
+    permT, l1, l2 = wsbb_amd.random_nodes(n, N, n + m)
+    idx = np.r_[0:200, N - 200:N, np.random.default_rng(7).choice(N, 1500, replace=False)]
+    ref = oracle.Oracle(p).bound_batch(permT[:, idx], l1[idx], l2[idx], threads=8)
+    with wsbb_amd.Engine(p) as eng:
+        assert np.array_equal(eng.bound(permT, l1, l2)[idx], ref)

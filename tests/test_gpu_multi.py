@@ -143,3 +143,27 @@ def test_plain_batches_by_class(sizes, counts):
             assert st["nodes"] == N * reps and st["fallbacks"] == 0
             assert st["pairs"] == reps * sum(c * p.shape[0] * (p.shape[0] - 1) // 2
                                              for c, p in zip(counts, ps))
+
+
+@pytest.mark.parametrize("sizes,per", [([(50, 5), (48, 6), (33, 8)], 44_001), ([(96, 5), (95, 7)], 50_003),
+                                       ([(70, 9), (94, 10)], 70_001)])
+def test_plain_batches_of_large_classes(sizes, per):
+    """Classes large enough for 128-node tiles (two row tiles, and three with
+    four column blocks) and one that stays on 64 (three row tiles)."""
+    rng = np.random.default_rng(per)
+    ps = [rng.integers(1, 100, size=(m, n)).astype(np.int32) for n, m in sizes]
+    maxn, N = max(n for n, _ in sizes), per * len(ps)
+    permT = np.zeros((maxn, N), np.uint8)
+    l1, l2 = np.zeros(N, np.int32), np.zeros(N, np.int32)
+    off = np.arange(len(ps) + 1, dtype=np.int32) * per
+    for i, p in enumerate(ps):
+        at, n = slice(off[i], off[i + 1]), p.shape[1]
+        permT[:n, at], l1[at], l2[at] = wsbb_amd.random_nodes(n, per, 100 + i)
+    with wsbb_amd.Multi(ps) as mb:
+        mb.load(permT, l1, l2, off)
+        got, _, _ = mb.run()
+    for i, p in enumerate(ps):
+        n = p.shape[1]
+        idx = off[i] + np.r_[0:200, per - 200:per, rng.choice(per, 800, replace=False)]
+        ref = oracle.Oracle(p).bound_batch(np.ascontiguousarray(permT[:n, idx]), l1[idx], l2[idx], threads=8)
+        assert np.array_equal(got[idx], ref)

@@ -234,3 +234,81 @@ def test_parents_at_the_edges_of_lane_groups(n, m, high):
     assert np.array_equal(np.concatenate([r["permT"].T for r in rounds]), tk["perm"].astype(np.uint8))
     for key in ("l1", "l2", "cost"):
         assert np.array_equal(np.concatenate([r[key] for r in rounds]), tk[key])
+
+
+def check_bounds(o, rnd, n):
+    permT, l1, l2 = rebuild_children(rnd, n)
+    ref = o.bound_batch(permT, l1, l2, threads=8)
+    bad = np.flatnonzero(ref != rnd["bound"])
+    assert bad.size == 0, (rnd["round"], bad[:5], ref[bad[:5]], rnd["bound"][bad[:5]])
+
+
+@pytest.mark.parametrize("n,m,topk,margin,parents", [
+    (20, 10, 6, -1, True), (20, 10, 6, 25, True), (20, 7, 4, 25, False), (20, 5, 10, -1, True),
+    (50, 9, 5, -1, True), (50, 6, 15, 40, True), (100, 5, 3, 60, False), (33, 13, 20, -1, True)])
+def test_learned_rounds_bound_the_same_in_both_forms(n, m, topk, margin, parents):
+    """A learned search on the matrix cores (subsets, and the listed children
+    within the margin) and by the scans, whose subset bounds are checked
+    against the oracle on batches: every round's parents and every child's
+    bound are equal.  With every pair selected they are the oracle's LB2."""
+    p = np.random.default_rng(n * m).integers(1, 100, size=(m, n)).astype(np.int32)
+    o = oracle.Oracle(p)
+    runs = []
+    for int16 in (1, 2):
+        with wsbb_amd.Engine(p) as eng:
+            eng.set_int16(int16)
+            eng.selector_init(seed=3)
+            eng.selector_config(topk=topk, margin=margin, parents=parents)
+            rounds = eng.search_trace()
+            res = eng.solve(kind=wsbb_amd.LEARNED, pool_size=3000, max_batches=3, budget=1500)
+            eng.search_trace(False)
+            runs.append((res, rounds))
+    (ra, a), (rb, b) = runs
+    assert ra["best"] == rb["best"] and ra["stats"] == rb["stats"]
+    assert len(a) == len(b) > 1 and any(r["desc"].shape[0] % 64 for r in a)
+    for x, y in zip(a, b):
+        for key in ("permT", "l1", "l2", "desc", "bound"):
+            assert np.array_equal(x[key], y[key]), (x["round"], key)
+        if topk == m * (m - 1) // 2:
+            check_bounds(o, x, n)
+
+
+@pytest.mark.parametrize("n,m,high,pool,nb,int16", [
+    (20, 10, 300, 3000, 2, 0), (20, 10, 300, 65536, 4, 1), (50, 9, 300, 3000, 2, 1), (50, 9, 300, 3000, 2, 0),
+    (127, 4, 99, 3000, 2, 1), (128, 5, 99, 3000, 2, 0), (128, 3, 300, 3000, 2, 1)])
+def test_rounds_beyond_the_matrix_core_form(n, m, high, pool, nb, int16):
+    """Instances with times above a signed byte or more than 126 jobs search
+    by the scans, from the parents' state: every child's bound and the pop
+    order against the oracle."""
+    p = np.random.default_rng(n + high).integers(1, high + 1, size=(m, n)).astype(np.int32)
+    p[0, 0] = high
+    o = oracle.Oracle(p)
+    _, st, _, tr = o.solve_batched(pool_size=pool, max_batches=nb, budget=1200, trace=10_000)
+    res, rounds = traced_solve(p, pool, nb, int16=int16, budget=1200)
+    assert res["stats"]["bounded"] == st["bounded"] == sum(r["desc"].shape[0] for r in rounds)
+    tk = {k: v[:st["decomposed"]] for k, v in taken(tr).items()}
+    assert np.array_equal(np.concatenate([r["permT"].T for r in rounds]), tk["perm"].astype(np.uint8))
+    for key in ("l1", "l2", "cost"):
+        assert np.array_equal(np.concatenate([r[key] for r in rounds]), tk[key])
+    for rnd in rounds:
+        check_bounds(o, rnd, n)
+
+
+def test_learned_solve_beyond_the_matrix_core_form():
+    """Subset and listed bounds by the scans on an instance with times above
+    a signed byte: valid bounds, full LB2 within the margin, plain's optimum."""
+    p = np.random.default_rng(5).integers(1, 200, size=(5, 12)).astype(np.int32)
+    p[0, 0] = 199
+    o = oracle.Oracle(p)
+    with wsbb_amd.Engine(p) as eng:
+        plain = eng.solve(pool_size=3000, max_batches=2)
+        eng.selector_init(seed=3)
+        eng.selector_config(topk=3, margin=50, parents=True)
+        rounds = eng.search_trace()
+        res = eng.solve(kind=wsbb_amd.LEARNED, pool_size=3000, max_batches=2)
+        eng.search_trace(False)
+    assert plain["proven"] and res["proven"] and res["best"] == plain["best"]
+    assert res["stats"]["fallbacks"] > 0
+    for rnd in rounds:
+        permT, l1, l2 = rebuild_children(rnd, 12)
+        assert (rnd["bound"] <= o.bound_batch(permT, l1, l2, threads=8)).all()
