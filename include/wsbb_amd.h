@@ -169,20 +169,29 @@ int wsbb_timer_start(wsbb_ctx *ctx);
 int wsbb_timer_stop(wsbb_ctx *ctx, float *ms);
 
 /* ---- launch shape and autotuning --------------------------------------------
- * groups: waves that split the pairs of one 64-node tile (1, 2, 4, 8 or
- * 16; 8 and 16 apply to plain LB2 with at most 16 machines, else 4);
- * grid_blocks: cap on 256-thread blocks (0 = automatic).  wsbb_autotune
- * times every shape that differs for the instance's LB2 kernel (at most 15)
- * on a synthetic batch of N nodes and keeps the fastest for that kernel's
- * batches of that size class, search rounds excepted; shapes (groups,
+ * groups: waves that split the pairs of one 64-node tile (1, 2, 4, 8 or 16;
+ * 0 and 1: chosen by batch size).  Plain LB2 on the matrix cores splits over 4
+ * at most up to 32 jobs, 2 up to 64, and not above; of the scans (other
+ * instances, LB1, optional outputs, large batches of few pairs) 8 and 16
+ * apply to plain LB2 with at most 16 machines, else 4.
+ * grid_blocks: cap on the 256-thread blocks of a launch (0 = automatic).  The
+ * scans' blocks loop over tiles under it; the matrix cores' do not, so a batch
+ * of more blocks runs as several launches, one after the other.
+ * wsbb_autotune times every shape that differs for the instance's LB2 kernel
+ * (at most 15) on a synthetic batch of N nodes and keeps the fastest for that
+ * kernel's batches of that size class, search rounds excepted; shapes (groups,
  * grid_blocks) and times are written if non-NULL. */
 int wsbb_set_launch(wsbb_ctx *ctx, int groups, int grid_blocks);
 int wsbb_autotune(wsbb_ctx *ctx, int N, int reps, int32_t *shapes,
                   float *ms, int *count);
-/* Plain LB2 (no optional outputs, best = -1) may run two nodes per lane in
- * int16 halves when every bound value of the instance stays below 2^14:
- * mode 1 (default) for batches of at least 2 x 128 x (4 x CUs) nodes, 2 for
- * every batch, 0 never.  Both forms give identical values. */
+/* Plain LB2 (no optional outputs, best = -1) runs on the matrix cores where
+ * every time is at most 127, n <= 126 and every lag + p_a fits two signed
+ * bytes, large batches of few pairs excepted; else by scans: one node a lane
+ * in int32, or two in int16 halves when every bound value of the instance
+ * stays below 2^14.  mode 1 (default): the int16 scan for scanned batches of at
+ * least 2 x 128 x (4 x CUs) nodes; 2: for every batch whose instance allows it,
+ * in place of the matrix cores too; 0: never.  All forms give identical
+ * values. */
 int wsbb_set_int16(wsbb_ctx *ctx, int mode);
 
 /* ---- device-resident branch-and-bound -------------------------------------------

@@ -359,7 +359,8 @@ class Engine:
 
     def set_int16(self, mode):
         """Two nodes per lane in int16 halves for plain LB2: 0 never, 1 for
-        large batches (default), 2 whenever the instance fits."""
+        large batches that the matrix cores do not take (default), 2 whenever
+        the instance fits, in their place too."""
         _check(lib.wsbb_set_int16(self.h, int(mode)), "set_int16")
 
     def search_options(self, use_graph=-1, rounds_per_sync=-1):

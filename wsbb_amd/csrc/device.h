@@ -49,9 +49,10 @@ struct DevTables {
   const uint2* steps16;  // [P][n4] two-node form {job, (p_a - p_b mod 2^16)
                          // | (2^14 + lag + p_b) << 16}; pad = 0, plus 16
                          // zero steps; null when bound values may reach 2^14
-  const int4* mf;        // [P][row tiles][column blocks][64] matrix-core operands
-                         // of every pair's Johnson scan (johnson.hip), or null
-                         // when the instance's times do not fit them
+  const int4* mf;        // [2 couples + 8][row tiles][column blocks][64] matrix-core
+                         // operands of the pairs' Johnson scans, in couples
+                         // (johnson.hip), or null when the instance's times do
+                         // not fit them
   const int4* pf;        // [column blocks][64] the processing times, alike
   const int4* pr;        // [n] the processing times job-major, a byte each
 };

@@ -837,9 +837,9 @@ JohnsonShape johnson_shape(int n, int P, int N, int waves, bool subset, int num_
   const int simds = 4 * num_cus, tiles = (N + 63) / 64;
   // The pairs are split over waves while that still adds waves to SIMDs that
   // have few, and where a tile's pairs outweigh the heads and tails that the
-  // split leaves to one wave (us at G = 1 / 2 / 4: 20x20, 50 000 nodes 34 / 27
-  // / 25; 100 003 nodes 41 / 37 / 43; 300 000 nodes 83 / 85 / 109; 30x12,
-  // 100 000 nodes 24 / 28 / 34).
+  // split leaves to one wave (us a launch, back to back, at G = 1 / 2 / 4: 20x20,
+  // 50 000 nodes 34 / 27 / 25; 100 003 nodes 42 / 38 / 43; 300 000 nodes 89 / 89
+  // / 111; 30x12, 100 000 nodes 24 / 29 / 35).
   H.groups = waves > 0                               ? waves
              : tiles * H.rts < simds                 ? 4
              : tiles * H.rts < 2 * simds && P >= 128 ? 2
@@ -847,18 +847,19 @@ JohnsonShape johnson_shape(int n, int P, int N, int waves, bool subset, int num_
   H.groups = subset ? 1 : std::max(1, std::min(H.groups, 4 / H.rts));
   // Tiles of 128 nodes halve the fragments' way through the L1 and the scalar
   // work, for twice the registers: with two row tiles of jobs and more, from
-  // two waves per SIMD on (us for 64 / 128 nodes: 50x20, 65 536 nodes 56 / 66;
-  // 130 000 nodes 101 / 93; 2^20 nodes 654 / 600; 100x10, 65 521 nodes 70 /
-  // 55).  With one row tile a block holds four such tiles, whose start clocks
-  // and tails leave room in LDS for one wave per SIMD: 300 000 nodes, 20x20 83
-  // / 151, 32x20 115 / 182, 32x5 30 / 40; 2^20 nodes, 32x20 332 / 485, 32x5 79
-  // / 88 (at 262 017 nodes, whose blocks just fill the chip, 32x5 is 28 / 25).
-  // With three row tiles a block is one tile of three waves, two of which run
-  // its prefixes and then its suffixes while the third waits: 90 jobs, 131 072
-  // nodes, 5 machines 56 / 72, 20 machines 220 / 244; 2^20 nodes, 5 machines
-  // 380 / 520, 10 machines 600 / 787 (95 and 96 jobs, whose fourth column
-  // block holds the constants, have two waves per SIMD at 64 nodes too: 96
-  // jobs, 2^20 nodes, 5 machines 629 / 557, 10 machines 953 / 863).
+  // two waves per SIMD on (us for 64 / 128 nodes, back to back: 50x20, 65 536
+  // nodes 57 / 63; 90 000 nodes 73 / 88; 130 000 nodes 102 / 92; 2^20 nodes 670
+  // / 623; 100x10, 50 000 nodes 70 / 52; 65 521 nodes 72 / 54).  With one row
+  // tile a block holds four such tiles, whose start clocks and tails leave
+  // room in LDS for one wave per SIMD: 300 000 nodes, 32x20 115 / 182, 32x5 30
+  // / 40; 2^20 nodes, 32x20 332 / 485, 32x5 79 / 88 (at 262 017 nodes, whose
+  // blocks just fill the chip, 32x5 is 28 / 25).  With three row tiles a block
+  // is one tile of three waves, two of which run its prefixes and then its
+  // suffixes while the third waits: 90 jobs, 131 072 nodes, 5 machines 56 / 72,
+  // 20 machines 220 / 244; 2^20 nodes, 5 machines 380 / 520, 10 machines 600 /
+  // 787 (95 and 96 jobs, whose fourth column block holds the constants, have
+  // two waves per SIMD at 64 nodes too: 96 jobs, 2^20 nodes, 5 machines 629 /
+  // 557, 10 machines 953 / 863).
   const bool third_idle = H.rts == 3 && column_blocks(n) == 3;
   H.wide = !subset && H.rts >= 2 && !third_idle && H.groups == 1 &&
            static_cast<long long>((N + 127) / 128) * H.rts >= 2 * simds;
