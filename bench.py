@@ -18,7 +18,7 @@ with LB2 and LB1 on the GPU and by the CPU explorer), "config2" (ta011, 20x10,
 time-to-optimum with 4096-child pools: ten per round, and one per round as
 the reference launches them), "learned_20x20" and "learned_online" (20x20
 plain against learned pair selection), "mixed_batch" (64 instances of uneven
-size in one launch), "solve_50x20" (50x20 instances to proven optimum, plain
+size in one call), "solve_50x20" (50x20 instances to proven optimum, plain
 and learned, against the CPU explorer).  CPU baselines are the oracle (the C
 restatement of the reference CPU path) on this host, on one thread and on all
 host cores.
@@ -458,7 +458,7 @@ def bench_50x20(wsbb_amd, host, cpu=True, seeds=(1, 11, 25, 27, 38, 49, 51, 65, 
 
 def bench_mixed(wsbb_amd, budget=100_000_000, host=None):
     """64 instances, n in {20, 50, 100} x m in {5, 10, 20}, job-correlated
-    times, 16384 random nodes each, bounded together in one launch per pass
+    times, 16384 random nodes each, bounded together in one call per pass
     until `budget` nodes are bounded: plain LB2 and learned pair selection
     (one MLP per machine count, trained on records of a plain solve of the
     first instance of that size, top-k = max(4, P/8) pairs per tile) with
